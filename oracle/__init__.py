@@ -25,11 +25,15 @@ _U = ctypes.c_uint32
 _I64 = ctypes.c_int64
 
 
+def ref_sources_present() -> bool:
+    return os.path.isfile(os.path.join(REF_ROOT, "src", "core", "quant.cpp"))
+
+
 def build(with_ref: bool = True, dropin: bool = False) -> None:
     """Compiles liboracle.so, and _ref/libcllm_ref.so when the reference tree is present; with
     dropin (after cllm_inference_amd's libraries are built) also _ref/libengine_dropin.so."""
     targets = ["all"]
-    if with_ref and os.path.isdir(REF_ROOT):
+    if with_ref and ref_sources_present():
         targets.append("ref")
         if dropin:
             targets.append("dropin")

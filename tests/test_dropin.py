@@ -38,7 +38,8 @@ def _cxx() -> str:
     pytest.skip("no C++ compiler")
 
 
-@pytest.mark.skipif(not os.path.isdir(REF), reason="needs the reference tree")
+@pytest.mark.skipif(not os.path.isfile(os.path.join(REF, ENGINE_SOURCES[0])),
+                    reason="needs the reference tree")
 def test_reference_engine_links_against_libcllm_quant(tmp_path):
     assert os.path.exists(QUANT_SO), "build libcllm_quant.so first (__graft_entry__.build())"
     cxx = _cxx()
