@@ -173,6 +173,43 @@ __device__ __forceinline__ void store_tile(int n, int m, const float* __restrict
     write_out([&](int i, int r) { return acc[i][r]; });
 }
 
+// The MFMA work of N items (one block of weights against one token tile each), software
+// pipelined inside the wave: item i's fragment reads are issued an item ahead, and its MFMAs
+// run beside the VALU epilogue of item i - 1 (load(i), mma(i), fin(i) take compile-time-constant
+// i after unrolling and keep their state in buffers indexed by i & 1). Left to itself the
+// compiler waits for each LDS read right after it and reuses one accumulator, so every item
+// pays the LDS and the MFMA latency: with two waves per SIMD the gate/up GEMM of the 8B model
+// at 512 rows spent 44 % of its wave cycles in waits and took @A@ us against @B@ us now.
+// MF MFMAs and EP epilogue VALU operations per item.
+template <int N, int MF, int EP, class Load, class Mma, class Fin>
+__device__ __forceinline__ void pipelined(Load load, Mma mma, Fin fin) {
+    if constexpr (MF > 4) {  // two weight tiles per wave: no registers for a second item
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            load(i);
+            mma(i);
+            fin(i);
+        }
+        return;
+    }
+    load(0);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (i + 1 < N) load(i + 1);
+        mma(i);
+        if (i > 0) fin(i - 1);
+        __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);  // the next item's LDS reads
+#pragma unroll
+        for (int g = 0; g < MF; ++g) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);        // an MFMA
+            __builtin_amdgcn_sched_group_barrier(0x002, EP / MF, 0);  // VALU beside it
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    fin(N - 1);
+}
+
 }  // namespace
 
 // Up to kMaxSegs weight matrices of one type and K over one activation batch, in one launch
@@ -382,38 +419,56 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_q4k(Segs segs, uint32_t row_by
                     afr[t][1][1] = scaled8(q.z & 0xF0F0F0F0u, q.w & 0xF0F0F0F0u, s_hi, c_hi);
                 }
             }
-            auto block = [&]<int BLK, bool FRESH>() {
-                const int b = 2 * PC + BLK;  // block within the stage
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt) {
+            // items i = BLK * MT + mt: block 2 PC + BLK against token tile mt. The super-block's
+            // first block starts the scaled sums.
+            wh8 bf[2][2];
+            float dxv[3];
+            wf16 f[NT == 1 ? 2 : 1][NT];
+            constexpr int FB = NT == 1 ? 1 : 0;  // accumulator buffers - 1
+            pipelined<2 * MT, NT == 1 ? 2 : 8, 16 * NT>(
+                [&](int i) {
+                    const int b = 2 * PC + i / MT, mt = i % MT;  // b: block within the stage
                     const uint8_t* arow = cur + (mt * 32 + r32) * 256;
                     const int sw = r32 & 15;
-                    const wh8 b0 = *(const wh8*)(arow + (((4 * b + 2 * h) ^ sw) << 4));
-                    const wh8 b1 = *(const wh8*)(arow + (((4 * b + 2 * h + 1) ^ sw) << 4));
-                    const float dxv = *(const float*)(cur + C::OFF_DX + (mt * 32 + r32) * 16 + 4 * b);
+                    bf[i & 1][0] = *(const wh8*)(arow + (((4 * b + 2 * h) ^ sw) << 4));
+                    bf[i & 1][1] = *(const wh8*)(arow + (((4 * b + 2 * h + 1) ^ sw) << 4));
+                    dxv[i % 3] = *(const float*)(cur + C::OFF_DX + (mt * 32 + r32) * 16 + 4 * b);
+                },
+                [&](int i) {
 #pragma unroll
                     for (int t = 0; t < NT; ++t) {
-                        wf16 f = {};
-                        f = __builtin_amdgcn_mfma_f32_32x32x16_f16(afr[t][BLK][0], b0, f, 0, 0, 0);
-                        f = __builtin_amdgcn_mfma_f32_32x32x16_f16(afr[t][BLK][1], b1, f, 0, 0, 0);
+                        const wf16 zero = {};
+                        f[i & FB][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afr[t][i / MT][0], bf[i & 1][0], zero, 0, 0, 0);
+                        f[i & FB][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afr[t][i / MT][1], bf[i & 1][1], f[i & FB][t], 0, 0, 0);
+                    }
+                },
+                [&](int i) {
+                    const int mt = i % MT;
+                    const float dx = dxv[i % 3];
+#pragma unroll
+                    for (int t = 0; t < NT; ++t)
 #pragma unroll
                         for (int r = 0; r < 16; ++r)
-                            sacc[t][mt][r] = FRESH ? dxv * f[r] : fmaf(dxv, f[r], sacc[t][mt][r]);
-                    }
-                }
-            };
-            // the super-block's first block starts the scaled sums (PC is wave-uniform)
-            if (HALF == 0 && PC == 0)
-                block.template operator()<0, true>();
-            else
-                block.template operator()<0, false>();
-            block.template operator()<1, false>();
+                            sacc[t][mt][r] = HALF == 0 && PC == 0 && i < MT ? dx * f[i & FB][t][r]
+                                                                            : fmaf(dx, f[i & FB][t][r], sacc[t][mt][r]);
+                    // the sums are needed here: not sunk to where they are read next
+                    if constexpr (NT == 1) asm volatile("" : "+v"(sacc[0][mt]));
+                });
         };
-        // (a rolled loop: unrolled, the compiler interleaves the two block pairs and spills)
+        if constexpr (NT == 1) {
+#pragma unroll
+            for (int pc = 0; pc < 2; ++pc) {
+                __builtin_amdgcn_sched_barrier(0);  // the two block pairs' registers do not overlap
+                if (more) issue_part(s + 1, nxt, pc);
+                blocks(pc);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        } else {
 #pragma unroll 1
-        for (int pc = 0; pc < 2; ++pc) {
-            if (more) issue_part(s + 1, nxt, pc);
-            blocks(pc);
+            for (int pc = 0; pc < 2; ++pc) {
+                if (more) issue_part(s + 1, nxt, pc);
+                blocks(pc);
+            }
         }
 
         // The next stage's loads have landed before the scratch is read (an LDS read while
@@ -677,66 +732,78 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_q6k(const uint8_t* __restrict_
         const uint8_t* act = cur;
         const float* dxl = (const float*)(cur + C::OFF_DX);
 
-        auto block = [&]<bool FRESH>(int i) {
+        // The A operands of block i: 16 s_hi (q - 32) and s_lo (q - 32), both exact in fp16. A
+        // quant byte pair becomes 64 + q with q's nibble on top of the low byte and its two high
+        // bits in the high byte, under the exponent of 64; one FMA then takes off 96 s.
+        auto unpack = [&](int i, wh8 (&a1)[2], wh8 (&a2)[2]) {
             const wu4 ql = window16(2 * (i & 1) + h);
-            const uint32_t lsh = i >= 2 ? 4u : 0u;
-            // bits 2i, 2i+1 of every qh byte to bits 4, 5 of the same byte: a rotation right by
-            // 2i - 4 (mod 32); the bits it carries across bytes are masked off
-            const uint32_t rot = (uint32_t)(2 * i - 4) & 31u;
             const uint32_t qhv[4] = {qhb.x, qhb.y, qhb.z, qhb.w}, qlv[4] = {ql.x, ql.y, ql.z, ql.w};
-            uint32_t q6[4];
+            uint32_t lo[4], hi[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                q6[e] = ((qlv[e] >> lsh) & 0x0F0F0F0Fu) |
-                        (__builtin_amdgcn_alignbit(qhv[e], qhv[e], rot) & 0x30303030u);
+            for (int e = 0; e < 4; ++e) {
+                lo[e] = (i >= 2 ? qlv[e] : qlv[e] << 4) & 0xF0F0F0F0u;
+                hi[e] = ((qhv[e] >> (2 * i)) & 0x03030303u) | 0x54545454u;
+            }
             // scale of this lane's 16 values: sc[8 g + 2 i + h], local index 2 i + h
             const int si = 2 * i + h;
-            const uint32_t scw = si < 4 ? scx : scy;
+            const uint32_t scw = i < 2 ? scx : scy;
             const int sc = (int)(int8_t)((scw >> (8 * (si & 3))) & 0xFFu);
-            const int s_hi = sc >> 4, s_lo = sc & 15;
-            const wh2 off = {(_Float16)-1056.0f, (_Float16)-1056.0f};
-            const wh2 m1 = {(_Float16)(16 * s_hi), (_Float16)(16 * s_hi)};
-            const wh2 m2 = {(_Float16)s_lo, (_Float16)s_lo};
-            wh8 a1[2], a2[2];
+            const _Float16 s1 = (_Float16)(sc & ~15), s2 = (_Float16)(sc & 15);
+            const _Float16 k1 = s1 * (_Float16)-96.0f, k2 = s2 * (_Float16)-96.0f;
+            const wh2 m1 = {s1, s1}, m2 = {s2, s2}, c1 = {k1, k1}, c2 = {k2, k2};
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                const wh2 v0 = magic_pair(q6[2 * j], 0) + off, v1 = magic_pair(q6[2 * j], 1) + off;
-                const wh2 v2 = magic_pair(q6[2 * j + 1], 0) + off, v3 = magic_pair(q6[2 * j + 1], 1) + off;
-                const wh2 p0 = v0 * m1, p1 = v1 * m1, p2 = v2 * m1, p3 = v3 * m1;
-                const wh2 q0 = v0 * m2, q1 = v1 * m2, q2 = v2 * m2, q3 = v3 * m2;
+                wh2 v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    v[e] = __builtin_bit_cast(wh2, __builtin_amdgcn_perm(
+                        hi[2 * j + (e >> 1)], lo[2 * j + (e >> 1)], e & 1 ? 0x07030602u : 0x05010400u));
+                const wh2 p0 = __builtin_elementwise_fma(v[0], m1, c1), p1 = __builtin_elementwise_fma(v[1], m1, c1);
+                const wh2 p2 = __builtin_elementwise_fma(v[2], m1, c1), p3 = __builtin_elementwise_fma(v[3], m1, c1);
+                const wh2 q0 = __builtin_elementwise_fma(v[0], m2, c2), q1 = __builtin_elementwise_fma(v[1], m2, c2);
+                const wh2 q2 = __builtin_elementwise_fma(v[2], m2, c2), q3 = __builtin_elementwise_fma(v[3], m2, c2);
                 a1[j] = wh8{p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y};
                 a2[j] = wh8{q0.x, q0.y, q1.x, q1.y, q2.x, q2.y, q3.x, q3.y};
             }
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-                const int tok = mt * 32 + r32;
-                const uint8_t* arow = act + tok * 256;
-                const int sw = tok & 15;
-                const wh8 b0 = *(const wh8*)(arow + (((4 * i + 2 * h) ^ sw) << 4));
-                const wh8 b1 = *(const wh8*)(arow + (((4 * i + 2 * h + 1) ^ sw) << 4));
-                const float dxv = dxl[i * BM + tok];
-                wf16 f = {};
-                f = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1[0], b0, f, 0, 0, 0);
-                f = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1[1], b1, f, 0, 0, 0);
-                f = __builtin_amdgcn_mfma_f32_32x32x16_f16(a2[0], b0, f, 0, 0, 0);
-                f = __builtin_amdgcn_mfma_f32_32x32x16_f16(a2[1], b1, f, 0, 0, 0);
-                if constexpr (FRESH) {
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) sacc[mt][r] = dxv * f[r];
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) sacc[mt][r] = fmaf(dxv, f[r], sacc[mt][r]);
-                }
-            }
         };
-        if constexpr (GH == 0)
-            block.template operator()<true>(0);
-        else
-            block.template operator()<false>(0);
-        block.template operator()<false>(1);
+        // blocks 2 pc and 2 pc + 1; items it = (block within the pair) * MT + token tile, the
+        // second block unpacked beside the first one's last item
+        auto blocks = [&](int pc) {
+            wh8 a1[2][2], a2[2][2], bf[2][2];
+            float dxv[3];
+            wf16 f[2];
+            pipelined<2 * MT, 4, 16>(
+                [&](int it) {
+                    const int i = 2 * pc + it / MT, tok = (it % MT) * 32 + r32, sw = r32 & 15;
+                    if (it % MT == 0) unpack(i, a1[it / MT], a2[it / MT]);
+                    const uint8_t* arow = act + tok * 256;
+                    bf[it & 1][0] = *(const wh8*)(arow + (((4 * i + 2 * h) ^ sw) << 4));
+                    bf[it & 1][1] = *(const wh8*)(arow + (((4 * i + 2 * h + 1) ^ sw) << 4));
+                    dxv[it % 3] = dxl[i * BM + tok];
+                },
+                [&](int it) {
+                    const int u = it / MT;
+                    wf16 z = {};
+                    z = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1[u][0], bf[it & 1][0], z, 0, 0, 0);
+                    z = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1[u][1], bf[it & 1][1], z, 0, 0, 0);
+                    z = __builtin_amdgcn_mfma_f32_32x32x16_f16(a2[u][0], bf[it & 1][0], z, 0, 0, 0);
+                    f[it & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a2[u][1], bf[it & 1][1], z, 0, 0, 0);
+                },
+                [&](int it) {
+                    const int mt = it % MT;
+                    const float dx = dxv[it % 3];
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        sacc[mt][r] = GH == 0 && pc == 0 && it < MT ? dx * f[it & 1][r]
+                                                                    : fmaf(dx, f[it & 1][r], sacc[mt][r]);
+                    asm volatile("" : "+v"(sacc[mt]));  // not sunk past the stage's branches
+                });
+        };
+        blocks(0);
+        __builtin_amdgcn_sched_barrier(0);
         if (more) issue_stage.template operator()<1 - GH, 1>(s + 1, nxt);
-#pragma unroll 1
-        for (int i = 2; i < 4; ++i) block.template operator()<false>(i);
+        blocks(1);
+        __builtin_amdgcn_sched_barrier(0);
         if (more) wait_vm();
         if constexpr (GH == 1) {
             float dr[16];
@@ -939,10 +1006,8 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_b32(const uint8_t* __restrict_
 
         const uint8_t* act = cur;
         const float* dxl = (const float*)(cur + C::OFF_DX);
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            // A fragments: elements 16h + 8j + e of block b (K steps j = 0, 1)
-            wh8 afr[2];
+        // A fragments: elements 16h + 8j + e of block b (K steps j = 0, 1)
+        auto unpack = [&](int b, wh8 (&afr)[2]) {
             if constexpr (T == T_Q8_0) {
                 uint32_t u[4];
                 lds_unaligned<4>(wr, b * BS + 2 + 16 * h, u);
@@ -970,21 +1035,33 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_b32(const uint8_t* __restrict_
                 afr[0] = scaled8(q[0], q[1], one, c);
                 afr[1] = scaled8(q[2], q[3], one, c);
             }
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-                const int tok = mt * 32 + r32;
+        };
+        // items it = block * MT + token tile, each block unpacked beside the item before it
+        wh8 afr[2][2], bf[2][2];
+        float dxv[3];
+        wf16 f[2];
+        pipelined<4 * MT, 2, 32>(
+            [&](int it) {
+                const int b = it / MT, tok = (it % MT) * 32 + r32, sw = r32 & 15;
+                if (it % MT == 0) unpack(b, afr[b & 1]);
                 const uint8_t* arow = act + tok * 256;
-                const int sw = tok & 15;
-                const wh8 b0 = *(const wh8*)(arow + (((4 * b + 2 * h) ^ sw) << 4));
-                const wh8 b1 = *(const wh8*)(arow + (((4 * b + 2 * h + 1) ^ sw) << 4));
-                const float dxv = dxl[tok * 4 + b];
-                wf16 f = {};
-                f = __builtin_amdgcn_mfma_f32_32x32x16_f16(afr[0], b0, f, 0, 0, 0);
-                f = __builtin_amdgcn_mfma_f32_32x32x16_f16(afr[1], b1, f, 0, 0, 0);
+                bf[it & 1][0] = *(const wh8*)(arow + (((4 * b + 2 * h) ^ sw) << 4));
+                bf[it & 1][1] = *(const wh8*)(arow + (((4 * b + 2 * h + 1) ^ sw) << 4));
+                dxv[it % 3] = dxl[tok * 4 + b];
+            },
+            [&](int it) {
+                const wf16 zero = {};
+                f[it & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afr[(it / MT) & 1][0], bf[it & 1][0], zero, 0, 0, 0);
+                f[it & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afr[(it / MT) & 1][1], bf[it & 1][1], f[it & 1], 0, 0, 0);
+            },
+            [&](int it) {
+                const int b = it / MT, mt = it % MT;
+                const float dx = dxv[it % 3];
 #pragma unroll
-                for (int r = 0; r < 16; ++r) yacc[mt][r] = fmaf(dxv, dr[b][r] * f[r], yacc[mt][r]);
-            }
-        }
+                for (int r = 0; r < 16; ++r)
+                    yacc[mt][r] = fmaf(dx, dr[b][r] * f[it & 1][r], yacc[mt][r]);
+                asm volatile("" : "+v"(yacc[mt]));  // not sunk past the stage's branches
+            });
         if (more) wait_vm();
         __syncthreads();
     };
