@@ -179,7 +179,10 @@ __device__ __forceinline__ void store_tile(int n, int m, const float* __restrict
 // i after unrolling and keep their state in buffers indexed by i & 1). Left to itself the
 // compiler waits for each LDS read right after it and reuses one accumulator, so every item
 // pays the LDS and the MFMA latency: with two waves per SIMD the gate/up GEMM of the 8B model
-// at 512 rows spent 44 % of its wave cycles in waits and took @A@ us against @B@ us now.
+// spent 44 % of its wave cycles in waits. MI355X, cold weights, us, before and now (the
+// s_setprio of the 256 x 128 tiles included): Q4_K 14336 x 4096 at 512 rows 133 and 118, Q5_K
+// 141 and 118, Q4_K 4096 x 14336 at 384 rows 122 and 105, Q8_0 14336 x 4096 at 100 rows 71 and
+// 51, Q5_0 14336 x 4096 at 512 rows 262 and 170.
 // MF MFMAs and EP epilogue VALU operations per item.
 template <int N, int MF, int EP, class Load, class Mma, class Fin>
 __device__ __forceinline__ void pipelined(Load load, Mma mma, Fin fin) {
@@ -459,10 +462,21 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_q4k(Segs segs, uint32_t row_by
 #pragma unroll
             for (int pc = 0; pc < 2; ++pc) {
                 __builtin_amdgcn_sched_barrier(0);  // the two block pairs' registers do not overlap
+                // Two waves of the workgroup share a SIMD, which favours the older one: it ran
+                // ahead and waited a quarter of its time at the barrier for the other, which then
+                // issued alone. The wave that is behind gets the SIMD instead (256 x 128 tiles,
+                // 14336 x 4096 at 512 rows: 197 k cycles a tile without, 184 k with it).
+                if constexpr (W == 8) {
+                    if (pc == 0)
+                        __builtin_amdgcn_s_setprio(2);
+                    else
+                        __builtin_amdgcn_s_setprio(1);
+                }
                 if (more) issue_part(s + 1, nxt, pc);
                 blocks(pc);
             }
             __builtin_amdgcn_sched_barrier(0);
+            if constexpr (W == 8) __builtin_amdgcn_s_setprio(0);
         } else {
 #pragma unroll 1
             for (int pc = 0; pc < 2; ++pc) {
