@@ -26,6 +26,7 @@ struct Tuning {
     std::atomic<int> gemv_fused_rows{0};  // streamed GEMV batches quantized in-kernel up to this many rows
     std::atomic<int> attention_kind{0};   // attention: 0 planner, 1 split kernel, 2 MFMA kernel
     std::atomic<int> gemv_fp_wgs{0};  // one-row float-dot GEMV: 0 planner, 1-8 pipelined kernel at that many workgroups per CU, 9 per-row kernel
+    std::atomic<int> gemm_f{0};  // float-dot GEMM: 0 planner, 1-3 its tile shapes from 2 rows, 9 never
 };
 Tuning& tuning();
 
@@ -187,6 +188,11 @@ hipError_t launch_dequantize_span(uint32_t type, const uint8_t* src, int64_t n, 
 // activation rows x[m][k], as the reference's dequantize fallback computes it.
 bool gemv_f_supported(uint32_t type);
 hipError_t launch_gemv_f(uint32_t type, const uint8_t* w, int k, int n, int m, const float* x,
+                         const float* bias, float* y, hipStream_t stream);
+// The same contract for batches on split-operand bf16 MFMA (k_gemm_f.hip; k % 32 == 0), and
+// whether a batch takes it (launch_gemv_f then runs it).
+bool gemm_f_takes(uint32_t type, int k, int n, int m);
+hipError_t launch_gemm_f(uint32_t type, const uint8_t* w, int k, int n, int m, const float* x,
                          const float* bias, float* y, hipStream_t stream);
 hipError_t gemmw_workspace_init(void* part, size_t bytes, hipStream_t stream);
 bool gemmw_supported(uint32_t type);

@@ -384,6 +384,9 @@ const char* cllm_hip_matmul_plan(uint32_t type, int in_dim, int out_dim, int n_r
  *                  quantized inside its launch (0 = the default)
  *   "attention_kernel" 0 the default, 1 the sequence-split kernel, 2 the many-row MFMA kernel
  *                  (decode with fused RoPE always takes the split kernel)
+ *   "gemm_f"       float-dot batches: 0 the default, 1 to 3 the split-operand MFMA kernel's tile
+ *                  shapes (128 rows x 64 tokens, 64 x 32, 32 x 32) from 2 rows, 9 the GEMV
+ *                  kernels for every batch
  *   "gemv_fp_wgs"  one activation row of Q4_1 / Q5_1 / Q8_1 (float dot), rows of up to two
  *                  blocks per lane: 0 the default, 1 to 8 the pipelined row walk at that many
  *                  workgroups per CU, 9 the per-row kernel

@@ -1,0 +1,64 @@
+"""The split-operand MFMA kernel of the float-dot types (csrc/k_gemm_f.hip) against the 64-bit
+sums, on every tile shape: weight rows and tokens at the edges of tiles, K of an odd number of
+32-element units, of less than a 256-element chunk and of a chunk more than the waves share
+evenly. Bars as for the GEMV of these types (test_gpu_fdot.py)."""
+import numpy as np
+import pytest
+
+from cllm_inference_amd import synth as S
+from test_gpu_parity import check_close, _dev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shape", [1, 2, 3])
+@pytest.mark.parametrize("qt", list(S.FLOAT_DOT_TYPES))
+def test_split_operand_gemm_edges(gpu, orc, qt, shape):
+    step = max(S.BLOCK[qt], 32)
+    for n, units, m in ((1, 1, 8), (31, 3, 33), (33, 9, 2), (129, 5, 65), (70, 27, 31), (128, 8, 64)):
+        k = step * units
+        w = S.make_weight(qt, n, k, 7 * n + k)
+        x = S.make_activation(m, k, m + k, outliers=True)
+        bias = np.random.default_rng(n).standard_normal(n).astype(np.float32)
+        print("gemm_f", S.TYPE_NAMES[qt], "shape", shape, n, k, m, flush=True)
+        gpu.tune("gemm_f", shape)
+        try:
+            y = gpu.matmul_quant_dev(_dev(x), _dev(w), qt, _dev(bias), k, n).cpu().numpy()
+        finally:
+            gpu.tune("gemm_f")
+        exact, abs_sum = orc.matmul_f64(x, w, qt, bias, k, n, m)
+        yo = orc.matmul(x, w, qt, bias, k, n, m).reshape(m, n)
+        check_close(y, yo, exact, abs_sum, f"{S.TYPE_NAMES[qt]} shape {shape} {n}x{k} m{m}")
+
+
+@pytest.mark.parametrize("qt", list(S.FLOAT_DOT_TYPES))
+def test_split_operand_gemm_non_finite(gpu, orc, qt):
+    """Activations with infinities, NaN and values past the largest bf16 give the reference's
+    infinities and NaNs, and the rows beside them the values of a batch without them."""
+    k, n, m = 512, 40, 12
+    w = S.make_weight(qt, n, k, 3)
+    x = S.make_activation(m, k, 4)
+    clean = x.copy()
+    x[1, 5], x[4, 300], x[7, 17], x[9, 2] = np.inf, -np.inf, np.nan, 3.4e38
+    out = {}
+    for knob in (1, 2, 3):
+        gpu.tune("gemm_f", knob)
+        try:
+            out[knob] = gpu.matmul_quant_dev(_dev(x), _dev(w), qt, None, k, n).cpu().numpy()
+            if knob == 2:
+                beside = gpu.matmul_quant_dev(_dev(clean), _dev(w), qt, None, k, n).cpu().numpy()
+        finally:
+            gpu.tune("gemm_f")
+    ref = orc.matmul(x, w, qt, None, k, n, m).reshape(m, n)
+    for knob in (1, 2, 3):
+        y = out[knob]
+        for t in (1, 4, 7):
+            # a zero weight makes inf * 0 = NaN; the others keep the sign
+            assert np.array_equal(np.isnan(y[t]), np.isnan(ref[t])), (knob, t)
+            inf = np.isinf(ref[t])
+            assert np.array_equal(y[t][inf], ref[t][inf]), (knob, t)
+        fin = np.isfinite(ref[9])
+        assert np.array_equal(np.isfinite(y[9]), fin), knob
+        np.testing.assert_allclose(y[9][fin], ref[9][fin], rtol=1e-5)
+    rows = [t for t in range(m) if t not in (1, 4, 7, 9)]
+    assert np.array_equal(out[2][rows], beside[rows])
