@@ -649,14 +649,25 @@ bool use_small(uint32_t type, int k, int n, int m) {
     return m >= lo && m <= (type == T_Q8_0 ? 64 : 32);
 }
 
-// The MFMA kernels walk K in 256-element steps. Crossover from the GEMV (which streams the
+// The MFMA kernels walk K in 256-element steps (the weight-row kernel of the 32-element block
+// types in blocks: Q8_0 4864 x 896 at 512 rows took 383 us on 64 GEMV launches of 8 rows, now
+// 30). Crossover from the GEMV (which streams the
 // weights once per 8 activation rows) measured on MI355X: 16 rows for the types the
 // weight-row kernel has; 64 for the others (and for shapes past the weight-row kernel's 32-bit
 // offsets), whose int8 kernel only overtakes the GEMV there
 // (Q5_K 14336 x 4096: 155 us at 16 rows against ~50 us on the GEMV). A forced kernel choice
 // (the tuning knob gemm_kernel) takes the MFMA route from 16 rows for every type.
 bool use_mfma(uint32_t type, int k, int n, int m) {
-    if (k % 256 != 0 || !gemm_supported(type) || use_small(type, k, n, m)) return false;
+    // rows of the 32-element block types that are no multiple of 256: the weight-row kernel
+    // only (the others walk K in whole 256-element steps), where the GEMV needs a third launch
+    // of 8 rows, or a second on matrices of 32 M weights or more. MI355X, cold weights, us, GEMV
+    // against weight-row kernel: Q8_0 4864x896 at 16 rows 14.2 / 14.4, 512 rows 383 / 30; Q4_0
+    // 3000x1184 at 100 rows 74 / 27; Q5_0 12000x8224 at 32 rows 218 / 46 (12 rows: 74 / 45).
+    if (k % 256 != 0) {
+        const bool large = (int64_t)n * k >= (int64_t(32) << 20);
+        return m > (large ? 8 : 16) && !gemm_forced() && gemmw_takes_k(type, k) && gemmw_fits(type, k, n, m);
+    }
+    if (!gemm_supported(type) || use_small(type, k, n, m)) return false;
     if (gemm_forced()) return m >= kMfmaMinRows;
     if (!gemmw_supported(type) || !gemmw_fits(type, k, n, m)) return m >= 4 * kMfmaMinRows;
     if (m >= kMfmaMinRows) return true;
@@ -814,6 +825,18 @@ hipError_t run_gemv_f32(uint32_t type, const uint8_t* w, int k, int n, int m, co
     return launch_gemv(type, w, k, n, m, ws.qs, ws.sc, ws.bs, bias, y, stream, accumulate);
 }
 
+// Whether stream s is being captured into a graph: nothing may be allocated then. The routes
+// that calls with rows of k % 256 != 0 took before they had the weight-row kernel allocate less;
+// under capture those calls keep to what is there.
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return cap != hipStreamCaptureStatusNone;
+}
+
 // The per-stream workspace of the device entry points, grown to an m x k batch and to the
 // split-K region of an n-row MFMA call on it (n = 0: none).
 int stream_workspace(DeviceState* st, hipStream_t s, uint32_t type, int k, int n, int m,
@@ -822,8 +845,11 @@ int stream_workspace(DeviceState* st, hipStream_t s, uint32_t type, int k, int n
     auto& slot = st->dev_ws[s];
     if (!slot) slot = std::make_unique<Workspace>();
     HIP_TRY(slot->ensure(k, m, s));
-    if (n > 0 && (use_mfma(type, k, n, m) || use_small(type, k, n, m)))
-        HIP_TRY(slot->ensure_part(part_bytes_for(type, k, n, m), s));
+    if (n > 0 && (use_mfma(type, k, n, m) || use_small(type, k, n, m))) {
+        // (without room for its partial sums the weight-row kernel does not split K)
+        const size_t pb = part_bytes_for(type, k, n, m);
+        if (k % 256 == 0 || pb <= slot->part.cap || !capturing(s)) HIP_TRY(slot->ensure_part(pb, s));
+    }
     *out = slot.get();
     return CLLM_HIP_OK;
 }
@@ -1064,7 +1090,8 @@ int cllm_hip_gemv_q8_dev(const void* w, uint32_t type, int in_dim, int out_dim, 
     DeviceState* st;
     if ((rc = acquire(&st))) return rc;
     hipStream_t s = (hipStream_t)stream;
-    if (!use_mfma(type, in_dim, out_dim, n_rows) && !use_small(type, in_dim, out_dim, n_rows)) {
+    if ((!use_mfma(type, in_dim, out_dim, n_rows) && !use_small(type, in_dim, out_dim, n_rows)) ||
+        (in_dim % 256 != 0 && capturing(s))) {
         HIP_TRY(launch_gemv(type, (const uint8_t*)w, in_dim, out_dim, n_rows, qs, scales, bsums,
                             bias, y, s));
         return CLLM_HIP_OK;
@@ -1399,6 +1426,8 @@ int cllm_hip_matmul_quant_static_dev(const float* x, const void* w, uint32_t typ
         if (use_mfma(type, in_dim, out_dim, n_rows) || use_small(type, in_dim, out_dim, n_rows))
             pb = part_bytes_for(type, in_dim, out_dim, n_rows);
     }
+    // without room for the split-K region K stays whole (rows no multiple of 256 long)
+    if (in_dim % 256 != 0 && act + pb > kStaticScratchBytes) pb = 0;
     if (act + pb > kStaticScratchBytes)
         return set_err(CLLM_HIP_E_ARG,
                        "matmul_quant: %d rows of %d need %zu bytes of scratch, more than the %zu "
@@ -1458,7 +1487,9 @@ int cllm_hip_matmul_quant_residual_dev(const float* x, const void* w, uint32_t t
     hipStream_t s = (hipStream_t)stream;
     Workspace* ws = nullptr;
     if ((rc = stream_workspace(st, s, type, in_dim, out_dim, n_rows, &ws))) return rc;
-    if (has_kernel(type) && !use_mfma(type, in_dim, out_dim, n_rows) && !use_small(type, in_dim, out_dim, n_rows)) {
+    if (has_kernel(type) &&
+        ((!use_mfma(type, in_dim, out_dim, n_rows) && !use_small(type, in_dim, out_dim, n_rows)) ||
+         (in_dim % 256 != 0 && capturing(s)))) {
         // the GEMV adds into y in its epilogue
         HIP_TRY(run_gemv_f32(type, (const uint8_t*)w, in_dim, out_dim, n_rows, x, bias, y, ws->v, s,
                              true));

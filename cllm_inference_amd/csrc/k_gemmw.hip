@@ -864,16 +864,17 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_q6k(const uint8_t* __restrict_
 template <uint32_t T>
 constexpr int b32_bytes() { return T == T_Q8_0 ? Q8_0_BYTES : T == T_Q4_0 ? Q4_0_BYTES : Q5_0_BYTES; }
 
-template <uint32_t T, int W, int MT>
+template <uint32_t T, int W, int MT, bool ANY>
 struct CfgB {
     static constexpr int THREADS = 64 * W;
     static constexpr int BN = 32 * W;
     static constexpr int BM = 32 * MT;
     static constexpr int SROW = 4 * b32_bytes<T>();   // bytes per weight row per stage
-    static constexpr int SDW = SROW / 4;
+    static constexpr int LROW = SROW + (ANY ? 4 : 0);  // LDS bytes per weight row
+    static constexpr int SDW = LROW / 4;
     static constexpr int ACT = BM * 256;                // swizzled fp16, as for the K-quants
     static constexpr int DX = BM * 16 < 1024 ? 1024 : BM * 16;
-    static constexpr int WB = (BN * SROW + 255) / 256 * 256 + 64;  // + slack for the last lane's 5th dword
+    static constexpr int WB = (BN * LROW + 255) / 256 * 256 + 64;  // + slack for the last lane's 5th dword
     static constexpr int OFF_DX = ACT;
     static constexpr int OFF_W = OFF_DX + DX;
     static constexpr int STAGE = OFF_W + WB;
@@ -882,7 +883,7 @@ struct CfgB {
     static_assert(LDS <= 160 * 1024, "LDS budget");
     static constexpr int A_LOADS = ACT / 1024;
     static constexpr int A_SLOTS = (A_LOADS + W - 1) / W;
-    static constexpr int DX_LOADS = DX / 1024;
+    static constexpr int DX_LOADS = ANY ? BM * 16 / 256 : DX / 1024;
     static constexpr int DX_SLOTS = (DX_LOADS + W - 1) / W;
     static constexpr int W_DW = BN * SDW;               // weight dwords per stage
     static constexpr int W_LOADS = (W_DW + 63) / 64;    // 4-byte wave-loads
@@ -892,9 +893,9 @@ struct CfgB {
 // Bytes [o, o + 4 N) of an LDS row whose base is 4-byte aligned, o even: N + 1 aligned dword
 // reads and a funnel shift.
 template <int N>
-__device__ __forceinline__ void lds_unaligned(const uint8_t* row, int o, uint32_t (&out)[N]) {
-    const uint32_t* p = (const uint32_t*)(row + (o & ~3));
-    const uint32_t sh = (uint32_t)(o & 3);
+__device__ __forceinline__ void lds_unaligned(const uint8_t* row, uint32_t o, uint32_t (&out)[N]) {
+    const uint32_t* p = (const uint32_t*)(row + (o & ~3u));
+    const uint32_t sh = o & 3u;
     uint32_t v[N + 1];
 #pragma unroll
     for (int i = 0; i <= N; ++i) v[i] = p[i];
@@ -908,7 +909,7 @@ __device__ __forceinline__ uint32_t bits_to_byte_bit4(uint32_t x) {
     return ((x | (x << 7) | (x << 14) | (x << 21)) & 0x01010101u) << 4;
 }
 
-template <uint32_t T, int W, int MT>
+template <uint32_t T, int W, int MT, bool ANY>
 __global__ __launch_bounds__(64 * W) void k_gemmw_b32(const uint8_t* __restrict__ w,
                                                       uint32_t row_bytes, int k, int n, int m,
                                                       const _Float16* __restrict__ qh,
@@ -916,7 +917,7 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_b32(const uint8_t* __restrict_
                                                       const float* __restrict__ bias,
                                                       float* __restrict__ y, float* __restrict__ part,
                                                       int* __restrict__ counters, int split_stages) {
-    using C = CfgB<T, W, MT>;
+    using C = CfgB<T, W, MT, ANY>;
     constexpr int BM = C::BM;
     constexpr int BS = b32_bytes<T>();
     extern __shared__ __align__(16) uint8_t lds[];
@@ -936,8 +937,9 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_b32(const uint8_t* __restrict_
     const int nblk = lin / mb_count, mblk = lin - nblk * mb_count;
     const int n0 = nblk * C::BN, m0 = mblk * BM;
     const int nb = k / 32;
+    const int stages = (k + kKS - 1) / kKS;
     const int s_begin = blockIdx.y * split_stages;
-    const int s_end = min(s_begin + split_stages, k / kKS);
+    const int s_end = min(s_begin + split_stages, stages);
 
     // per-lane source offsets (stage 0); rows and tokens past the matrix are clamped
     uint32_t a_off[C::A_SLOTS];
@@ -946,40 +948,55 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_b32(const uint8_t* __restrict_
         const int L = min(wave + j * W, C::A_LOADS - 1);
         const int t = 4 * L + (lane >> 4);
         const int c = (lane & 15) ^ (t & 15);
-        a_off[j] = ((uint32_t)min(m0 + t, m - 1) * (uint32_t)k + 8u * (uint32_t)c) * 2u;
+        a_off[j] = ((uint32_t)min(m0 + t, m - 1) * (uint32_t)k + (ANY ? 0u : 8u * (uint32_t)c)) * 2u;
     }
+    // (ANY: the chunk's first element, the same in every slot of a lane: slots are 4 W tokens
+    // apart, and 4 W is a multiple of 16)
+    static_assert(!ANY || (4 * W) % 16 == 0, "one chunk per lane");
+    const uint32_t a_el = 8u * (uint32_t)((lane & 15) ^ ((4 * wave + (lane >> 4)) & 15));
     uint32_t dx_off[C::DX_SLOTS];
 #pragma unroll
     for (int j = 0; j < C::DX_SLOTS; ++j) {
-        const int t = min(wave + j * W, C::DX_LOADS - 1) * 64 + lane;
-        dx_off[j] = (uint32_t)min(m0 + t, m - 1) * (uint32_t)nb;
+        const int f = min(wave + j * W, C::DX_LOADS - 1) * 64 + lane;
+        dx_off[j] = (uint32_t)min(m0 + (ANY ? f >> 2 : f), m - 1) * (uint32_t)nb;
     }
     uint32_t w_off[C::W_SLOTS];   // flat dword f of [row][SDW]: row f / SDW, dword f % SDW
 #pragma unroll
     for (int j = 0; j < C::W_SLOTS; ++j) {
         const int f = min(min(wave + j * W, C::W_LOADS - 1) * 64 + lane, C::W_DW - 1);
         const int row = f / C::SDW, dw = f - row * C::SDW;
-        w_off[j] = (uint32_t)min(n0 + row, n - 1) * row_bytes + 4u * (uint32_t)dw;
+        const uint32_t base = (uint32_t)min(n0 + row, n - 1) * row_bytes;
+        w_off[j] = (ANY ? base & ~3u : base) + 4u * (uint32_t)dw;
     }
+    const uint32_t w_bytes = (uint32_t)n * row_bytes;
+    const uint32_t w_last = (w_bytes - 4u) & ~3u;  // ANY: the last whole dword
 
     auto issue_stage = [&](int s, uint8_t* st) {
 #pragma unroll
         for (int j = 0; j < C::A_SLOTS; ++j) {
             const int L = wave + j * W;
             if (C::A_LOADS % W == 0 || L < C::A_LOADS)
-                lds_load16((const uint8_t*)qh + a_off[j] + (uint32_t)s * (2u * kKS), st + L * 1024);
+                lds_load16((const uint8_t*)qh + a_off[j] +
+                               (ANY ? 2u * min((uint32_t)s * kKS + a_el, (uint32_t)k - 8u) : (uint32_t)s * (2u * kKS)),
+                           st + L * 1024);
         }
 #pragma unroll
         for (int j = 0; j < C::DX_SLOTS; ++j) {
             const int L = wave + j * W;
-            if (C::DX_LOADS % W == 0 || L < C::DX_LOADS)
-                lds_load16(xs + dx_off[j] + (uint32_t)s * 4, st + C::OFF_DX + L * 1024);
+            if (C::DX_LOADS % W == 0 || L < C::DX_LOADS) {
+                if constexpr (ANY)
+                    lds_load4(xs + dx_off[j] + min(4 * s + (lane & 3), nb - 1), st + C::OFF_DX + L * 256);
+                else
+                    lds_load16(xs + dx_off[j] + (uint32_t)s * 4, st + C::OFF_DX + L * 1024);
+            }
         }
 #pragma unroll
         for (int j = 0; j < C::W_SLOTS; ++j) {
             const int L = wave + j * W;
             if (C::W_LOADS % W == 0 || L < C::W_LOADS)
-                lds_load4(w + w_off[j] + (uint32_t)s * (uint32_t)C::SROW, st + C::OFF_W + L * 256);
+                lds_load4(w + (ANY ? min(w_off[j] + (uint32_t)s * (uint32_t)C::SROW, w_last)
+                                   : w_off[j] + (uint32_t)s * (uint32_t)C::SROW),
+                          st + C::OFF_W + L * 256);
         }
     };
 
@@ -991,12 +1008,24 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_b32(const uint8_t* __restrict_
 
     float* scratch = (float*)(lds + 2 * C::STAGE) + wave * 128;
     const int wrow = wave * 32 + r32;
+    // ANY: the lead of this lane's row window, 0 or 2 bytes
+    const uint32_t sh = ANY ? ((uint32_t)min(n0 + wrow, n - 1) * row_bytes) & 2u : 0u;
+    // ANY: the half dword at the end of the matrix (its row, n - 1, starts at a multiple of 4)
+    const bool half_dword = ANY && (w_bytes & 2u) && n0 + C::BN >= n;
+    auto patch = [&](int s, uint8_t* st) {
+        if (!half_dword || s != stages - 1) return;
+        if (threadIdx.x == 0) {
+            const uint32_t at = w_bytes - 2u - ((uint32_t)(n - 1) * row_bytes + (uint32_t)s * (uint32_t)C::SROW);
+            *(uint16_t*)(st + C::OFF_W + (n - 1 - n0) * C::LROW + at) = *(const uint16_t*)(w + w_bytes - 2u);
+        }
+        __syncthreads();
+    };
 
     auto run_stage = [&](int s) {
         const int buf = (s - s_begin) & 1;
         uint8_t* cur = lds + buf * C::STAGE;
         uint8_t* nxt = lds + (1 - buf) * C::STAGE;
-        const uint8_t* wr = cur + C::OFF_W + wrow * C::SROW;
+        const uint8_t* wr = cur + C::OFF_W + wrow * C::LROW;
 
         // d of blocks 2h and 2h + 1 of this lane's row -> scratch, then each lane's 16 output
         // rows' d for all 4 blocks into registers, before the next stage's direct-to-LDS loads
@@ -1004,8 +1033,10 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_b32(const uint8_t* __restrict_
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             const int b = 2 * h + e;
-            const uint32_t dw = *(const uint32_t*)(wr + ((b * BS) & ~3));
-            scratch[b * 32 + r32] = f16_to_f32(((b * BS) & 2) ? (dw >> 16) : (dw & 0xFFFFu));
+            const uint32_t at = (uint32_t)(b * BS) + sh;
+            const uint32_t dw = *(const uint32_t*)(wr + (at & ~3u));
+            const float dv = f16_to_f32((at & 2u) ? (dw >> 16) : (dw & 0xFFFFu));
+            scratch[b * 32 + r32] = ANY && 4 * s + b >= nb ? 0.0f : dv;
         }
         float dr[4][16];
 #pragma unroll
@@ -1024,16 +1055,16 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_b32(const uint8_t* __restrict_
         auto unpack = [&](int b, wh8 (&afr)[2]) {
             if constexpr (T == T_Q8_0) {
                 uint32_t u[4];
-                lds_unaligned<4>(wr, b * BS + 2 + 16 * h, u);
+                lds_unaligned<4>(wr, (uint32_t)(b * BS + 2 + 16 * h) + sh, u);
                 afr[0] = __builtin_bit_cast(wh8, int8x8_to_h8(u[0], u[1]));
                 afr[1] = __builtin_bit_cast(wh8, int8x8_to_h8(u[2], u[3]));
             } else {
                 uint32_t u[4], hb = 0;
                 if constexpr (T == T_Q4_0) {
-                    lds_unaligned<4>(wr, b * BS + 2, u);
+                    lds_unaligned<4>(wr, (uint32_t)(b * BS + 2) + sh, u);
                 } else {
                     uint32_t v[5];
-                    lds_unaligned<5>(wr, b * BS + 2, v);
+                    lds_unaligned<5>(wr, (uint32_t)(b * BS + 2) + sh, v);
                     hb = v[0] >> (16 * h);
                     u[0] = v[1]; u[1] = v[2]; u[2] = v[3]; u[3] = v[4];
                 }
@@ -1078,12 +1109,14 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_b32(const uint8_t* __restrict_
             });
         if (more) wait_vm();
         __syncthreads();
+        if (more) patch(s + 1, nxt);
     };
 
     if (s_begin < s_end) {
         issue_stage(s_begin, lds);
         wait_vm();
         __syncthreads();
+        patch(s_begin, lds);
         for (int s = s_begin; s < s_end; ++s) run_stage(s);
     }
 
@@ -1105,6 +1138,8 @@ bool gemmw_fits(uint32_t type, int k, int n, int m) {
 }
 
 bool is_b32(uint32_t type) { return type == T_Q8_0 || type == T_Q4_0 || type == T_Q5_0; }
+
+bool gemmw_takes_k(uint32_t type, int k) { return gemmw_supported(type) && k % (is_b32(type) ? 32 : 256) == 0; }
 
 namespace {
 
@@ -1274,22 +1309,23 @@ hipError_t launch_q6(const uint8_t* w, int k, int n, int m, const _Float16* qh, 
     return hipGetLastError();
 }
 
-template <uint32_t T, int W, int MT>
+template <uint32_t T, int W, int MT, bool ANY>
 hipError_t launch_b32(const uint8_t* w, int k, int n, int m, const _Float16* qh, const float* xs,
                       const float* bias, float* y, float* part, int* counters, int splits,
                       hipStream_t stream) {
-    using C = CfgB<T, W, MT>;
+    using C = CfgB<T, W, MT, ANY>;
     static bool attr_set = false;
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void*)k_gemmw_b32<T, W, MT>,
+        hipError_t e = hipFuncSetAttribute((const void*)k_gemmw_b32<T, W, MT, ANY>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
         if (e != hipSuccess) return e;
         attr_set = true;
     }
     const uint32_t row_bytes = (uint32_t)(k / 32) * (uint32_t)b32_bytes<T>();
     const int tiles = ((n + C::BN - 1) / C::BN) * ((m + C::BM - 1) / C::BM);
-    const int stages = k / kKS, per = 2 * ((stages / 2 + splits - 1) / splits);
-    hipLaunchKernelGGL((k_gemmw_b32<T, W, MT>), dim3((unsigned)tiles, (unsigned)splits),
+    const int stages = (k + kKS - 1) / kKS;
+    const int per = k % 256 == 0 ? 2 * ((stages / 2 + splits - 1) / splits) : (stages + splits - 1) / splits;
+    hipLaunchKernelGGL((k_gemmw_b32<T, W, MT, ANY>), dim3((unsigned)tiles, (unsigned)splits),
                        dim3(C::THREADS), C::LDS, stream, w, row_bytes, k, n, m, qh, xs, bias, y, part,
                        counters, per);
     return hipGetLastError();
@@ -1314,7 +1350,7 @@ constexpr size_t kCounterBytes = 64 * 1024;  // 16384 tiles
 size_t gemmw_counter_bytes() { return kCounterBytes; }
 
 size_t gemmw_partial_bytes(uint32_t type, int k, int n, int m) {
-    if (!gemmw_supported(type) || k % 256 != 0) return 0;
+    if (!gemmw_takes_k(type, k)) return 0;
     const Plan p = plan_for(type, k, n, m);
     return p.splits > 1 ? slices_bytes(p, n, m) + kCounterBytes : 0;
 }
@@ -1353,7 +1389,7 @@ int segs_rows(const Segs& sg) {
 hipError_t gemmw_dispatch(uint32_t type, const Segs& sg, int k, int m, const float* xs,
                           const _Float16* qh, const uint16_t* xq, float* part, size_t part_bytes,
                           hipStream_t stream) {
-    if (!gemmw_supported(type) || k % 256 != 0 || sg.count < 1 || sg.count > kMaxSegs)
+    if (!gemmw_takes_k(type, k) || sg.count < 1 || sg.count > kMaxSegs)
         return hipErrorNotSupported;
     if (sg.count > 1 && type != T_Q4_K && type != T_Q5_K) return hipErrorNotSupported;
     for (int i = 0; i < sg.count; ++i)
@@ -1384,10 +1420,14 @@ hipError_t gemmw_dispatch(uint32_t type, const Segs& sg, int k, int m, const flo
     } else if (is_b32(type)) {
 #define CLLM_GEMMW_B32(TT)                                                                    \
         if (type == TT) {                                                                      \
-            if (p.mt == 2)                                                                     \
-                e = launch_b32<TT, 4, 2>(w, k, n, m, qh, xs, bias, y, part, counters, p.splits, stream); \
+            if (k % kKS != 0 && p.mt == 2)                                                     \
+                e = launch_b32<TT, 4, 2, true>(w, k, n, m, qh, xs, bias, y, part, counters, p.splits, stream); \
+            else if (k % kKS != 0)                                                             \
+                e = launch_b32<TT, 4, 1, true>(w, k, n, m, qh, xs, bias, y, part, counters, p.splits, stream); \
+            else if (p.mt == 2)                                                                \
+                e = launch_b32<TT, 4, 2, false>(w, k, n, m, qh, xs, bias, y, part, counters, p.splits, stream); \
             else                                                                               \
-                e = launch_b32<TT, 4, 1>(w, k, n, m, qh, xs, bias, y, part, counters, p.splits, stream); \
+                e = launch_b32<TT, 4, 1, false>(w, k, n, m, qh, xs, bias, y, part, counters, p.splits, stream); \
         }
         CLLM_GEMMW_B32(T_Q8_0)
         CLLM_GEMMW_B32(T_Q4_0)
@@ -1477,7 +1517,7 @@ void gemmw_multi_plan_name(uint32_t type, int k, int count, const int* n, int m,
 }
 
 void gemmw_plan_name(uint32_t type, int k, int n, int m, char* buf, size_t cap) {
-    if (!gemmw_supported(type) || k % 256 != 0) {
+    if (!gemmw_takes_k(type, k)) {
         snprintf(buf, cap, "none");
         return;
     }

@@ -123,7 +123,7 @@ hipError_t launch_gemm16(uint32_t type, const uint8_t* w, int k, int n, int m,
 
 // The weight-row fp16-MFMA GEMM (k_gemmw.hip), same contract as launch_gemm, on the activation
 // format of launch_quantize_w: dx (xs), fp16 values (qh) and, for Q4_K, the minimum operand
-// (xq). All six types; k % 256 == 0. When its plan splits K it needs a workspace part of at
+// (xq). All six types; k % 256 == 0 (the 32-element block types: k % 32 == 0). When its plan splits K it needs a workspace part of at
 // least gemmw_partial_bytes(type, k, n, m) bytes (else K is not split), zeroed once by
 // gemmw_workspace_init when allocated: the splits write partial sums there and the last split
 // of each tile adds them into y inside the same launch.
@@ -196,6 +196,9 @@ hipError_t launch_gemm_f(uint32_t type, const uint8_t* w, int k, int n, int m, c
                          const float* bias, float* y, hipStream_t stream);
 hipError_t gemmw_workspace_init(void* part, size_t bytes, hipStream_t stream);
 bool gemmw_supported(uint32_t type);
+// whether the weight-row kernels take rows of k elements of the type: whole super-blocks of the
+// K-quants, whole blocks of the 32-element block types
+bool gemmw_takes_k(uint32_t type, int k);
 // Several matrices of one type and K over one activation batch in one weight-row launch
 // (Q4_K / Q5_K, up to 3): the same contract as launch_gemmw per matrix, the split-K region
 // sized by gemmw_multi_partial_bytes.

@@ -1,0 +1,68 @@
+"""The weight-row kernel of the 32-element block types on rows that are no multiple of 256
+elements (csrc/k_gemmw.hip, k_gemmw_b32): whole stages of 128 in an odd number, a last stage of
+one to three blocks, rows that start at 2-byte alignment, a matrix that ends in half a dword (an
+odd number of rows of an odd number of blocks), and K splits; against the oracle, and against the
+GEMV the calls keep to under graph capture."""
+import numpy as np
+import pytest
+
+from cllm_inference_amd import synth as S
+from test_gpu_parity import check_close, _dev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("splits", [0, 2, 3])
+@pytest.mark.parametrize("qt", [S.Q8_0, S.Q4_0, S.Q5_0])
+def test_rows_of_whole_blocks(gpu, orc, qt, splits):
+    for n, k, m in ((300, 896, 100), (1, 32, 17), (129, 416, 33), (255, 2080, 64), (131, 1120, 17),
+                    (128, 1056, 31), (257, 160, 65), (64, 4000, 18)):
+        if splits > (k + 127) // 128:
+            continue
+        w = S.make_weight(qt, n, k, n + k)
+        x = S.make_activation(m, k, m, outliers=True)
+        bias = np.random.default_rng(k).standard_normal(n).astype(np.float32)
+        gpu.tune("gemm_splits", splits)
+        try:
+            print("k32", S.TYPE_NAMES[qt], n, k, m, gpu.matmul_plan(qt, k, n, m), flush=True)
+            assert gpu.matmul_route(qt, k, n, m) == "mfma"
+            y = gpu.matmul_quant_dev(_dev(x), _dev(w), qt, _dev(bias), k, n).cpu().numpy()
+            res = _dev(np.ones((m, n), np.float32))
+            if n % 4 == 0:
+                gpu.matmul_quant_residual_dev(_dev(x), _dev(w), qt, _dev(bias), k, n, res)
+        finally:
+            gpu.tune("gemm_splits")
+        exact, abs_sum = orc.matmul_f64(x, w, qt, bias, k, n, m)
+        yo = orc.matmul(x, w, qt, bias, k, n, m)
+        check_close(y, yo, exact, abs_sum, f"{S.TYPE_NAMES[qt]} {n}x{k} m{m} splits={splits}")
+        if n % 4 == 0:
+            assert np.array_equal(res.cpu().numpy(), 1.0 + y)
+
+
+def test_rows_of_whole_blocks_under_capture(gpu, orc):
+    """A captured call with nothing warmed up but the activation workspace, replayed between eager
+    work, equals the eager result."""
+    import torch
+    qt, n, k, m = S.Q8_0, 300, 2080, 48
+    w, x = S.make_weight(qt, n, k, 1), S.make_activation(m, k, 2, outliers=True)
+    wd, xd = _dev(w), _dev(x)
+    eager = gpu.matmul_quant_dev(xd, wd, qt, None, k, n).clone()
+    y = torch.zeros((m, n), device="cuda")
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        gpu.quantize_q8_0_dev(xd)
+        gpu.matmul_quant_dev(xd[:15], wd, qt, None, k, n)  # a GEMV batch: no room for split sums
+        gpu.matmul_quant_dev(torch.cat([xd, xd]), wd, S.Q8_0, None, k, 1)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        gpu.matmul_quant_dev(xd, wd, qt, None, k, n, y=y)
+    exact, abs_sum = orc.matmul_f64(x, w, qt, None, k, n, m)
+    yo = orc.matmul(x, w, qt, None, k, n, m)
+    for rep in range(3):
+        y.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        check_close(y.cpu().numpy(), yo, exact, abs_sum, f"replay {rep}")
+        again = gpu.matmul_quant_dev(xd, wd, qt, None, k, n)
+        assert torch.equal(again, eager)
