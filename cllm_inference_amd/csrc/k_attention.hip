@@ -13,14 +13,9 @@
 // k_attention_mfma (many query rows, on fp32 MFMA; its layout is described above it).
 //
 // Attention layout. One workgroup per (KV head, query row, sequence split); it serves the
-// n_rep query heads of that KV head, so every K and V row is loaded once for all of them.
-// Positions go in chunks of 64: sixteen lanes per position read the K row (16-byte pieces,
-// coalesced), each lane dots its slice with every query head held in registers, a 16-lane
-// reduction gives the scores; the softmax is online (running max and sum per head, the
-// partial output rescaled when the max grows); each wave adds p_t v_t for its 16 positions
-// of the chunk into per-lane partial outputs (lane l owns dims l + 64 e of every head), with
-// every K and V load of a chunk issued before the arithmetic that needs it; the four waves'
-// partials are added at the end.
+// n_rep query heads of that KV head, so every K and V row is loaded once for all of them. Its
+// waves walk the positions on their own (the layout is described at the kernel); the softmax is
+// online (running max and sum, the partial output rescaled when the max grows).
 // Long sequences are split over several workgroups whose (max, sum, unnormalised output)
 // partials the last of them to finish combines (a per-(row, KV head) arrival counter), so a
 // decode step (one query row) still spreads over the device in one launch. The summation
@@ -77,20 +72,81 @@ constexpr int kMaxSplits = 256;      // sequence splits per (row, KV head)
 // (two floats of padding keep every row 16-byte aligned for the combine's vector loads).
 // With one split, the normalised output goes straight to out.
 //
+// Waves work alone: no barrier and no LDS between the query's staging and the end. A wave
+// takes 4 P positions at a time, P in each of its four 16-lane rows; lane seg of a row holds
+// dims 64 i + 4 seg .. + 3 (i < HD / 64) of the K row, the V row, every query head of the group
+// and every head's output (a load instruction reads 256 contiguous bytes of four cache rows).
+// The P NREP scores of a row's positions are reduced together: each DPP step halves the number
+// of values a lane still carries, so lane idx(j, r) ends with the score of position j and head
+// r, takes its exponential once, and hands it to the row by a DPP broadcast. Maxima and sums
+// are per row of lanes (and head); the 16 rows of the workgroup meet at the end.
+//
+// What bounds it: the cache stream. One chunk of 64 positions per step with three barriers and
+// a reduction per (position, head) took 54 us over 8192 positions of 8 KV heads (67 MB) and
+// 15 us over 1024; this form takes 23 and 11.5, of which 9 go to the launch, the rotation and
+// the meeting of the splits (MI355X, 32 query heads of 128).
+//
+// (Nontemporal loads of the cache rows measured slower: 31.7 against 24.8 us at 8192.)
+//
 // rope_base > 0 (one query row, a decode step): the queries and the key row at pos0 arrive
 // unrotated and the kernel applies the NEOX rotation of k_rope_neox itself, to the queries in
 // registers and to the key row as it loads it, writing the rotated key row back to k_new (the
-// cache row pos0, read by no other workgroup: only the split holding pos0 covers it). k_new
-// points into the key cache, so kc carries no __restrict__: the compiler may not treat the
-// cache as unwritten by this kernel.
-template <int HD>
-__global__ __launch_bounds__(kThreads) void k_attention(
+// cache row pos0, read by no other workgroup: only the split holding pos0 covers it; waves of
+// this workgroup that clamp to it mask its score). k_new points into the key cache, so kc
+// carries no __restrict__: the compiler may not treat the cache as unwritten by this kernel.
+template <int CTRL>
+__device__ __forceinline__ float row_bcast(float v) { return dpp_f32<0x150 + CTRL>(v); }
+// the value of lane LANE of each 16-lane row (LANE constant after unrolling)
+__device__ __forceinline__ float bcast16(float v, int lane) {
+    switch (lane) {
+        case 0: return row_bcast<0>(v);
+        case 1: return row_bcast<1>(v);
+        case 2: return row_bcast<2>(v);
+        case 3: return row_bcast<3>(v);
+        case 4: return row_bcast<4>(v);
+        case 5: return row_bcast<5>(v);
+        case 6: return row_bcast<6>(v);
+        case 7: return row_bcast<7>(v);
+        case 8: return row_bcast<8>(v);
+        case 9: return row_bcast<9>(v);
+        case 10: return row_bcast<10>(v);
+        case 11: return row_bcast<11>(v);
+        case 12: return row_bcast<12>(v);
+        case 13: return row_bcast<13>(v);
+        case 14: return row_bcast<14>(v);
+        default: return row_bcast<15>(v);
+    }
+}
+
+// One step of the joint reduction over a 16-lane row: lanes whose bit is clear keep the first
+// half of the values, the others the second, each plus the partner's.
+template <int CTRL, int V>
+__device__ __forceinline__ void halve(float (&v)[V], int n, bool upper) {
+#pragma unroll
+    for (int i = 0; i < V / 2; ++i) {
+        if (i >= n / 2) break;
+        const float keep = upper ? v[i + n / 2] : v[i], give = upper ? v[i] : v[i + n / 2];
+        v[i] = keep + dpp_f32<CTRL>(give);
+    }
+}
+
+// Positions per lane row and step: as many as leave registers for two waves per SIMD (one at
+// head_dim 256 with 8 heads), at most 16 scores.
+template <int HD, int NREP>
+constexpr int attention_p() { return HD == 256 ? (NREP == 8 ? 1 : NREP == 4 ? 2 : 4) : NREP == 8 ? 2 : 4; }
+
+template <int HD, int NREP>
+__global__ __launch_bounds__(kThreads, HD == 256 && NREP == 8 ? 1 : 2) void k_attention(
     const float* __restrict__ q, const float* kc, const float* __restrict__ vc,
     int n_head, int n_kv, int pos0, int split_len, float scale, float* __restrict__ part,
     int* __restrict__ counters, float* __restrict__ out, float rope_base, float* k_new) {
-    constexpr int PER = HD / kLanesPerPos;  // K elements per lane (4 .. 16)
-    __shared__ float sc[kMaxRep][kChunk];
-    __shared__ float m_run[kMaxRep], l_run[kMaxRep], corr[kMaxRep];
+    constexpr int PER = HD / kLanesPerPos;   // dims per lane (4, 8 or 16)
+    constexpr int NB = PER / 4;              // 16-byte pieces per lane and row
+    constexpr int P = attention_p<HD, NREP>();  // positions per lane row and step
+    constexpr int V = P * NREP;              // scores per lane row and step (4, 8 or 16)
+    constexpr int DUP = 16 / V;              // lanes that end with the same score
+    constexpr int STEP = 4 * P;
+    constexpr int W = kThreads / 64;
 
     const int kvh = blockIdx.x, t = blockIdx.y, z = blockIdx.z, S = gridDim.z;
     const int n_rep = n_head / n_kv;
@@ -99,189 +155,200 @@ __global__ __launch_bounds__(kThreads) void k_attention(
     const int begin = z * split_len;
     const int end = min(L, begin + split_len);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int seg = lane % kLanesPerPos, sub = lane / kLanesPerPos;  // sub: position in wave
+    const int seg = lane & 15, sub = lane >> 4;
 
-    // this lane's slice of every query head of the group
-    float qv[kMaxRep][PER];
+    const float* kg = kc + (size_t)kvh * HD + 4 * seg;
+    const float* vg = vc + (size_t)kvh * HD + 4 * seg;
+    float kf[P][PER], vf[P][PER];
+    // position c0 + 4 j + sub, clamped to the split's last (its score is then masked)
+    auto load = [&](float (&x)[P][PER], const float* base, int c0) {
 #pragma unroll
-    for (int r = 0; r < kMaxRep; ++r) {
-        const float* qh = q + ((size_t)t * n_head + kvh * n_rep + min(r, n_rep - 1)) * HD + seg * PER;
+        for (int j = 0; j < P; ++j) {
+            const float* row = base + (size_t)min(c0 + 4 * j + sub, end - 1) * kv_dim;
 #pragma unroll
-        for (int e = 0; e < PER; e += 4) {
-            const f32x4 v = *(const f32x4*)(qh + e);
-            qv[r][e] = v.x; qv[r][e + 1] = v.y; qv[r][e + 2] = v.z; qv[r][e + 3] = v.w;
-        }
-    }
-    // NEOX rotation at position pos0: dims seg * PER + e pair with the partner lane seg ^ 8
-    // (the other half of the head); lanes seg < 8 hold x0 (dims i < HD / 2), the others x1.
-    const bool rope = rope_base > 0.0f;
-    const bool lo_half = seg < 8;
-    float rc[PER], rs[PER];
-    auto rotate = [&](float (&x)[PER]) {
-#pragma unroll
-        for (int e = 0; e < PER; ++e) {
-            const float other = __shfl_xor(x[e], 8, 16);
-            const float x0 = lo_half ? x[e] : other, x1 = lo_half ? other : x[e];
-            x[e] = lo_half ? __builtin_fmaf(x0, rc[e], -__fmul_rn(x1, rs[e]))
-                           : __builtin_fmaf(x0, rs[e], __fmul_rn(x1, rc[e]));
+            for (int i = 0; i < NB; ++i) {
+                const f32x4 v = *(const f32x4*)(row + 64 * i);
+                x[j][4 * i] = v.x; x[j][4 * i + 1] = v.y; x[j][4 * i + 2] = v.z; x[j][4 * i + 3] = v.w;
+            }
         }
     };
-    // the angles of the HD / 2 pairs, one per thread, shared through LDS
+    float qv[NREP][PER];
+#pragma unroll
+    for (int r = 0; r < NREP; ++r) {
+        const float* qh = q + ((size_t)t * n_head + kvh * n_rep + min(r, n_rep - 1)) * HD + 4 * seg;
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            const f32x4 v = *(const f32x4*)(qh + 64 * i);
+            qv[r][4 * i] = v.x; qv[r][4 * i + 1] = v.y; qv[r][4 * i + 2] = v.z; qv[r][4 * i + 3] = v.w;
+        }
+    }
+    // (after the queries: loads return in order, and the queries are rotated first)
+    int c0 = begin + wave * STEP;
+    load(kf, kg, c0);
+    load(vf, vg, c0);
+    // NEOX rotation at position pos0: dim i pairs with i + HD / 2, held by the same lane (HD >=
+    // 128) or by lane seg ^ 8 (HD = 64). The angles of the pairs, one per thread, go through LDS.
+    const bool rope = rope_base > 0.0f;
     __shared__ float rope_cs[2][HD / 2];
-    if (rope && threadIdx.x < HD / 2) {
-        const int i = threadIdx.x;
-        const float theta = __fdiv_rn((float)pos0, powf(rope_base, __fdiv_rn((float)i, (float)(HD / 2))));
-        rope_cs[0][i] = cosf(theta);
-        rope_cs[1][i] = sinf(theta);
-    }
-    // Each wave accumulates the output of its own 16 positions of every chunk: lane l owns
-    // dims l + 64 e (e < HD / 64) of every query head of the group; the four waves' partials
-    // are added at the end.
-    constexpr int DE = HD / 64;
-    float acc[kMaxRep][DE];
-#pragma unroll
-    for (int r = 0; r < kMaxRep; ++r)
-#pragma unroll
-        for (int e = 0; e < DE; ++e) acc[r][e] = 0.0f;
-    if (threadIdx.x < kMaxRep) {
-        m_run[threadIdx.x] = -INFINITY;
-        l_run[threadIdx.x] = 0.0f;
-    }
-    __syncthreads();
-    if (rope) {
+    float rc[PER], rs[PER];
+    auto rotate = [&](float (&x)[PER]) {
+        float o[PER];
 #pragma unroll
         for (int e = 0; e < PER; ++e) {
-            rc[e] = rope_cs[0][(seg & 7) * PER + e];
-            rs[e] = rope_cs[1][(seg & 7) * PER + e];
+            const bool lo = HD == 64 ? seg < 8 : e < PER / 2;
+            const float other = HD == 64 ? dpp_f32<0x128>(x[e]) : x[(e + PER / 2) % PER];  // row_ror:8
+            const float x0 = lo ? x[e] : other, x1 = lo ? other : x[e];
+            o[e] = lo ? __builtin_fmaf(x0, rc[e], -__fmul_rn(x1, rs[e]))
+                      : __builtin_fmaf(x0, rs[e], __fmul_rn(x1, rc[e]));
         }
 #pragma unroll
-        for (int r = 0; r < kMaxRep; ++r) rotate(qv[r]);
+        for (int e = 0; e < PER; ++e) x[e] = o[e];
+    };
+    if (rope) {
+        if (threadIdx.x < HD / 2) {
+            const int i = threadIdx.x;
+            const float theta = __fdiv_rn((float)pos0, powf(rope_base, __fdiv_rn((float)i, (float)(HD / 2))));
+            rope_cs[0][i] = cosf(theta);
+            rope_cs[1][i] = sinf(theta);
+        }
+        // a barrier that orders LDS only: the cache rows stay in flight
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+#pragma unroll
+        for (int e = 0; e < PER; ++e) {
+            const int d = (64 * (e >> 2) + 4 * seg + (e & 3)) % (HD / 2);
+            rc[e] = rope_cs[0][d];
+            rs[e] = rope_cs[1][d];
+        }
+#pragma unroll
+        for (int r = 0; r < NREP; ++r) rotate(qv[r]);
     }
 
-    for (int c0 = begin; c0 < end; c0 += kChunk) {
-        // scores of the chunk: each wave takes 4 positions per round, 4 rounds; all the K
-        // loads of the chunk are issued before the first dot
-        float kv[kChunk / 16][PER];
+    float acc[NREP][PER];
 #pragma unroll
-        for (int round = 0; round < kChunk / 16; ++round) {
-            const int pc = min(c0 + round * 16 + wave * 4 + sub, end - 1);
-            const float* kr = kc + (size_t)pc * kv_dim + kvh * HD + seg * PER;
+    for (int r = 0; r < NREP; ++r)
 #pragma unroll
-            for (int e = 0; e < PER; e += 4) {
-                const f32x4 v = *(const f32x4*)(kr + e);
-                kv[round][e] = v.x; kv[round][e + 1] = v.y; kv[round][e + 2] = v.z;
-                kv[round][e + 3] = v.w;
-            }
-        }
-        // the new key row (clamped positions past the end repeat it, and rotate it alike)
-        bool knew[kChunk / 16];
-        if (rope) {
+        for (int e = 0; e < PER; ++e) acc[r][e] = 0.0f;
+    // running maximum and sum of this lane's head (lanes with the same head agree)
+    float m_run = -INFINITY, l_run = 0.0f;
+    const int my_j = seg / DUP / NREP;  // the position of a step whose score this lane ends with
+
+    for (; c0 < end; c0 += W * STEP) {
+        if (rope && c0 <= pos0 && pos0 < c0 + STEP) {  // the new key row
 #pragma unroll
-            for (int round = 0; round < kChunk / 16; ++round) {
-                knew[round] = min(c0 + round * 16 + wave * 4 + sub, end - 1) == pos0;
+            for (int j = 0; j < P; ++j) {
                 float rot[PER];
 #pragma unroll
-                for (int e = 0; e < PER; ++e) rot[e] = kv[round][e];
+                for (int e = 0; e < PER; ++e) rot[e] = kf[j][e];
                 rotate(rot);
-                if (knew[round]) {
+                if (c0 + 4 * j + sub == pos0) {
+                    float* kw = k_new + kvh * HD + 4 * seg;
 #pragma unroll
-                    for (int e = 0; e < PER; ++e) kv[round][e] = rot[e];
+                    for (int i = 0; i < NB; ++i) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) kf[j][4 * i + e] = rot[4 * i + e];
+                        *(f32x4*)(kw + 64 * i) = f32x4{rot[4 * i], rot[4 * i + 1], rot[4 * i + 2], rot[4 * i + 3]};
+                    }
                 }
             }
         }
-        // this wave's V rows, issued with the K rows so both latencies overlap the score and softmax
-        // work (rows past the end are clamped, their probability is zero)
-        float vv[16][DE];
+        float s[V];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int pc = min(c0 + wave * 16 + j, end - 1);
-            const float* vr = vc + (size_t)pc * kv_dim + kvh * HD + lane;
+        for (int j = 0; j < P; ++j)
 #pragma unroll
-            for (int e = 0; e < DE; ++e) vv[j][e] = vr[64 * e];
-        }
-#pragma unroll
-        for (int round = 0; round < kChunk / 16; ++round) {
-            const int slot = round * 16 + wave * 4 + sub;
-            const int p = c0 + slot;
-#pragma unroll
-            for (int r = 0; r < kMaxRep; ++r) {
-                if (r >= n_rep) break;
+            for (int r = 0; r < NREP; ++r) {
                 float d = 0.0f;
 #pragma unroll
-                for (int e = 0; e < PER; ++e) d = __builtin_fmaf(qv[r][e], kv[round][e], d);
-                d += __shfl_xor(d, 8, 16);
-                d += __shfl_xor(d, 4, 16);
-                d += __shfl_xor(d, 2, 16);
-                d += __shfl_xor(d, 1, 16);
-                if (seg == 0) sc[r][slot] = p < end ? __fmul_rn(d, scale) : -INFINITY;
+                for (int e = 0; e < PER; ++e) d = __builtin_fmaf(qv[r][e], kf[j][e], d);
+                s[j * NREP + r] = d;
             }
+        // (loads of the next step, past the split's last one clamped in bounds and not used)
+        load(kf, kg, min(c0 + W * STEP, end - 1));
+        // lanes seg ^ 8, seg ^ 7 (a half row's mirror), seg ^ 2, seg ^ 1: together the 16 lanes
+        halve<0x128, V>(s, V, seg & 8);
+        halve<DPP_ROW_HALF_MIRROR, V>(s, V / 2, seg & 4);
+        if constexpr (V >= 8) halve<DPP_QUAD_SWAP2, V>(s, V / 4, seg & 2);
+        else s[0] += dpp_f32<DPP_QUAD_SWAP2>(s[0]);
+        if constexpr (V >= 16) halve<DPP_QUAD_SWAP1, V>(s, V / 8, seg & 1);
+        else s[0] += dpp_f32<DPP_QUAD_SWAP1>(s[0]);
+        const float sv = c0 + 4 * my_j + sub < end ? __fmul_rn(s[0], scale) : -INFINITY;
+        // the same head's lanes: seg ^ 8 (two positions) and seg ^ 4 (four)
+        float mx = sv;
+        if constexpr (P >= 2) mx = fmaxf(mx, dpp_f32<0x128>(mx));
+        if constexpr (P == 4) mx = fmaxf(mx, dpp_f32<0x1B>(dpp_f32<DPP_ROW_HALF_MIRROR>(mx)));
+        const float mn = fmaxf(m_run, mx);
+        const float pr = sv == -INFINITY ? 0.0f : expf(sv - mn);
+        const float cr = m_run == -INFINITY ? 0.0f : expf(m_run - mn);
+        float ps = pr;
+        if constexpr (P >= 2) ps += dpp_f32<0x128>(ps);
+        if constexpr (P == 4) ps += dpp_f32<0x1B>(dpp_f32<DPP_ROW_HALF_MIRROR>(ps));
+        m_run = mn;
+        l_run = __builtin_fmaf(l_run, cr, ps);
+#pragma unroll
+        for (int r = 0; r < NREP; ++r) {
+            const float c = bcast16(cr, r * DUP);
+#pragma unroll
+            for (int e = 0; e < PER; ++e) acc[r][e] *= c;
         }
-        __syncthreads();
-        // every K load of the workgroup has been consumed: the rotated row can go back
-        if (rope) {
 #pragma unroll
-            for (int round = 0; round < kChunk / 16; ++round) {
-                if (knew[round]) {
-                    float* kw = k_new + kvh * HD + seg * PER;
+        for (int j = 0; j < P; ++j)
 #pragma unroll
-                    for (int e = 0; e < PER; e += 4)
-                        *(f32x4*)(kw + e) = f32x4{kv[round][e], kv[round][e + 1], kv[round][e + 2], kv[round][e + 3]};
-                }
+            for (int r = 0; r < NREP; ++r) {
+                const float p = bcast16(pr, (j * NREP + r) * DUP);
+#pragma unroll
+                for (int e = 0; e < PER; ++e) acc[r][e] = __builtin_fmaf(p, vf[j][e], acc[r][e]);
             }
-        }
-        // one wave per query head (lane i = position i of the chunk): the running max, the
-        // probabilities relative to it in place of the scores, their sum, and the factor that
-        // rescales what is already summed
-        static_assert(kChunk == 64, "a chunk is one wave's lanes");
-        for (int r = wave; r < n_rep; r += kThreads / 64) {
-            const float s = sc[r][lane];
-            float cm = s;
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) cm = fmaxf(cm, __shfl_xor(cm, o, 64));
-            const float mo = m_run[r], mn = fmaxf(mo, cm);
-            const float pr = s == -INFINITY ? 0.0f : expf(s - mn);
-            float ps = pr;
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) ps += __shfl_xor(ps, o, 64);
-            sc[r][lane] = pr;
-            if (lane == 0) {
-                const float cr = mo == -INFINITY ? 0.0f : expf(mo - mn);
-                corr[r] = cr;
-                m_run[r] = mn;
-                l_run[r] = __builtin_fmaf(l_run[r], cr, ps);
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < kMaxRep; ++r) {
-            if (r >= n_rep) break;
-            const float cr = corr[r];
-#pragma unroll
-            for (int e = 0; e < DE; ++e) {
-                float a = acc[r][e] * cr;
-#pragma unroll
-                for (int j = 0; j < 16; ++j) a = __builtin_fmaf(sc[r][wave * 16 + j], vv[j][e], a);
-                acc[r][e] = a;
-            }
-        }
-        __syncthreads();
+        load(vf, vg, min(c0 + W * STEP, end - 1));
     }
 
-    // the four waves' partial outputs, added through LDS (reusing nothing else: a separate
-    // buffer), then the split's partial or the normalised output
-    __shared__ float wpart[kThreads / 64][kMaxRep * HD];
+    // The 16 lane rows' partials: maxima and sums through LDS, each row's output scaled to the
+    // common maximum, the four rows of a wave added across its lanes, the four waves through LDS.
+    __shared__ float wpart[W][NREP * HD];
+    __shared__ float mrow[4 * W][NREP], lrow[4 * W][NREP], m_all[NREP], l_all[NREP];
+    if (seg < NREP * DUP && seg % DUP == 0) {
+        mrow[wave * 4 + sub][seg / DUP] = m_run;
+        lrow[wave * 4 + sub][seg / DUP] = l_run;
+    }
+    __syncthreads();
+    if (threadIdx.x < NREP) {
+        const int r = threadIdx.x;
+        float M = -INFINITY, l = 0.0f;
 #pragma unroll
-    for (int r = 0; r < kMaxRep; ++r) {
+        for (int i = 0; i < 4 * W; ++i) M = fmaxf(M, mrow[i][r]);
+#pragma unroll
+        for (int i = 0; i < 4 * W; ++i) {
+            const float m = mrow[i][r], e = expf(m - M);
+            const float w = m == -INFINITY ? 0.0f : e;
+            l = __builtin_fmaf(w, lrow[i][r], l);
+            mrow[i][r] = w;
+        }
+        m_all[r] = M;
+        l_all[r] = l;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < NREP; ++r) {
         if (r >= n_rep) break;
+        const float w = mrow[wave * 4 + sub][r];
 #pragma unroll
-        for (int e = 0; e < DE; ++e) wpart[wave][r * HD + lane + 64 * e] = acc[r][e];
+        for (int i = 0; i < NB; ++i) {
+            float o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                o[e] = acc[r][4 * i + e] * w;
+                o[e] += __shfl_xor(o[e], 16, 64);
+                o[e] += __shfl_xor(o[e], 32, 64);
+            }
+            if (sub == 0) *(f32x4*)&wpart[wave][r * HD + 64 * i + 4 * seg] = f32x4{o[0], o[1], o[2], o[3]};
+        }
     }
     __syncthreads();
     if (S == 1) {
         for (int o = threadIdx.x; o < n_rep * HD; o += kThreads) {
             const int r = o / HD, d = o - r * HD;
             const float v = (wpart[0][o] + wpart[1][o]) + (wpart[2][o] + wpart[3][o]);
-            out[((size_t)t * n_head + kvh * n_rep + r) * HD + d] = __fdiv_rn(v, l_run[r]);
+            out[((size_t)t * n_head + kvh * n_rep + r) * HD + d] = __fdiv_rn(v, l_all[r]);
         }
         return;
     }
@@ -295,8 +362,8 @@ __global__ __launch_bounds__(kThreads) void k_attention(
         float* pp = part + (((size_t)t * n_head + kvh * n_rep + r) * S + z) * (HD + 4);
         __hip_atomic_store(pp + d, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (d == 0) {
-            __hip_atomic_store(pp + HD, m_run[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(pp + HD + 1, l_run[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(pp + HD, m_all[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(pp + HD + 1, l_all[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
     __builtin_amdgcn_s_waitcnt(0);  // this thread's partial stores have completed
@@ -310,80 +377,98 @@ __global__ __launch_bounds__(kThreads) void k_attention(
     }
     __syncthreads();
     if (!last) return;
-    // out = sum_z e^(m_z - M) o_z / sum_z e^(m_z - M) l_z, per head of the group. The maxima
-    // and sums of all splits are loaded at once (one per thread) into LDS; each output then
-    // reads its S values sixteen loads at a time.
-    auto ld = [](const float* a) {
-        return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    };
-    __shared__ float wz[kMaxRep][kMaxSplits], lsum[kMaxRep];
-    float* mz = &wpart[0][0];  // the wave partials are consumed: reuse as [kMaxRep][S] maxima
-    for (int i = threadIdx.x; i < n_rep * S; i += kThreads) {
-        const int r = i / S, zz = i - r * S;
-        const float* pz = part + (((size_t)t * n_head + kvh * n_rep + r) * S + zz) * (HD + 4);
-        mz[r * S + zz] = ld(pz + HD);
-        wz[r][zz] = ld(pz + HD + 1);  // the sums for now
-    }
-    __syncthreads();
-    if (threadIdx.x < n_rep) {
-        const int r = threadIdx.x;
-        float M = -INFINITY;
-        for (int zz = 0; zz < S; ++zz) M = fmaxf(M, mz[r * S + zz]);
-        float den = 0.0f;
-        for (int zz = 0; zz < S; ++zz) {
-            const float m = mz[r * S + zz];
-            const float wgt = m == -INFINITY ? 0.0f : expf(m - M);
-            den = __builtin_fmaf(wgt, wz[r][zz], den);
-            wz[r][zz] = wgt;
-        }
-        lsum[r] = den;
-    }
-    __syncthreads();
-    // Each thread takes four consecutive dims of one head and reads them as one 16-byte
-    // load per split: a buffer load with the SC1 bit, the same device-scope cache policy as
-    // the agent-scope atomic loads above, over this (row, KV head)'s partial rows. Sixteen
-    // splits at a time are in flight; per output the additions are in split order.
+    // out = sum_z e^(m_z - M) o_z / sum_z e^(m_z - M) l_z, per head of the group.
+    //
+    // Each thread takes four consecutive dims of one head over one of G ranges of the splits
+    // and reads them as one 16-byte load per split: a buffer load with the SC1 bit, the same
+    // device-scope cache policy as the agent-scope atomic loads below, over this (row, KV
+    // head)'s partial rows. Sixteen splits at a time are in flight, the first sixteen beside the
+    // maxima and sums; the ranges are added through LDS in order (the wave partials are consumed).
     typedef float f32x4v __attribute__((ext_vector_type(4)));
     const float* pg = part + ((size_t)t * n_head + kvh * n_rep) * S * (HD + 4);
     const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(
         (void*)pg, (short)0, (int)((size_t)n_rep * S * (HD + 4) * sizeof(float)), 0x00020000);
-    auto ld4 = [&](uint32_t off) {
-        return __builtin_bit_cast(f32x4v, __builtin_amdgcn_raw_buffer_load_b128(prs, off, 0, 16));
-    };
     constexpr int Q = HD / 4;
-    for (int o = threadIdx.x; o < n_rep * Q; o += kThreads) {
-        const int r = o / Q, d = 4 * (o - r * Q);
-        const uint32_t off0 = (uint32_t)((r * S * (HD + 4) + d) * sizeof(float));
-        const uint32_t zstep = (uint32_t)((HD + 4) * sizeof(float));
+    const int outs = n_rep * Q;
+    const int G = outs <= kThreads / 4 ? 4 : outs <= kThreads / 2 ? 2 : 1;
+    const int zlen = (S + G - 1) / G;
+    auto ld16 = [&](int o, int zz, uint32_t lead, f32x4v (&v)[16]) {  // (offsets past the rows read as zero)
+        const int gi = o / outs, oo = o - gi * outs;
+        const int r = oo / Q, d = 4 * (oo - r * Q), z1 = min(S, (gi + 1) * zlen);
+        const uint32_t off = (uint32_t)(((r * S + gi * zlen + zz) * (HD + 4) + d) * sizeof(float)) + lead;
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+            v[u] = __builtin_bit_cast(f32x4v, __builtin_amdgcn_raw_buffer_load_b128(
+                prs, gi * zlen + zz + u < z1 ? off + u * (uint32_t)((HD + 4) * sizeof(float)) : 0x7FFFFFF0u, 0, 16));
+    };
+    uint32_t lead = 0;  // opaque: the loads stay behind the branch above
+    asm volatile("" : "+v"(lead));
+    f32x4v first[16];
+    ld16(min((int)threadIdx.x, outs * G - 1), 0, lead, first);
+    // a wave per head turns the splits' maxima and sums into weights, 64 splits at a time
+    auto ld = [](const float* a) {
+        return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    __shared__ float wz[NREP][kMaxSplits + 16];
+    constexpr int ZR = kMaxSplits / 64;
+    for (int r = wave; r < n_rep; r += W) {
+        const float* pz = part + ((size_t)t * n_head + kvh * n_rep + r) * S * (HD + 4);
+        float m[ZR], l[ZR], M = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < ZR; ++i) {
+            const int zz = 64 * i + lane;
+            m[i] = zz < S ? ld(pz + (size_t)zz * (HD + 4) + HD) : -INFINITY;
+            l[i] = zz < S ? ld(pz + (size_t)zz * (HD + 4) + HD + 1) : 0.0f;
+            M = fmaxf(M, m[i]);
+        }
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
+        float den = 0.0f;
+#pragma unroll
+        for (int i = 0; i < ZR; ++i) {
+            const float e = expf(m[i] - M);
+            const float w = m[i] == -INFINITY ? 0.0f : e;
+            if (64 * i + lane < S) wz[r][64 * i + lane] = w;
+            den = __builtin_fmaf(w, l[i], den);
+        }
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) den += __shfl_xor(den, o, 64);
+        if (lane == 0) l_all[r] = den;
+    }
+    __syncthreads();
+    for (int o = threadIdx.x; o < outs * G; o += kThreads) {
+        const int gi = o / outs, oo = o - gi * outs;
+        const int r = oo / Q, d = 4 * (oo - r * Q);
         f32x4v num = {0.0f, 0.0f, 0.0f, 0.0f};
-        auto add = [&](float wgt, f32x4v v) {
-            num.x = __builtin_fmaf(wgt, v.x, num.x);
-            num.y = __builtin_fmaf(wgt, v.y, num.y);
-            num.z = __builtin_fmaf(wgt, v.z, num.z);
-            num.w = __builtin_fmaf(wgt, v.w, num.w);
-        };
-        int zz = 0;
-        for (; zz + 16 <= S; zz += 16) {
-            f32x4v v[16];
+        const int len = min(S, (gi + 1) * zlen) - gi * zlen;
+        for (int zz = 0; zz < len; zz += 16) {
+            if (zz > 0 || o >= kThreads) ld16(o, zz, 0, first);
 #pragma unroll
-            for (int u = 0; u < 16; ++u) v[u] = ld4(off0 + (uint32_t)(zz + u) * zstep);
-#pragma unroll
-            for (int u = 0; u < 16; ++u) add(wz[r][zz + u], v[u]);
+            for (int u = 0; u < 16; ++u) {
+                const float wgt = zz + u < len ? wz[r][gi * zlen + zz + u] : 0.0f;  // past the range: 0 * 0
+                num.x = __builtin_fmaf(wgt, first[u].x, num.x);
+                num.y = __builtin_fmaf(wgt, first[u].y, num.y);
+                num.z = __builtin_fmaf(wgt, first[u].z, num.z);
+                num.w = __builtin_fmaf(wgt, first[u].w, num.w);
+            }
         }
-        if (zz < S) {  // the last S % 16, also loaded together (one round trip, same order)
-            f32x4v v[16];
-#pragma unroll
-            for (int u = 0; u < 16; ++u)
-                v[u] = zz + u < S ? ld4(off0 + (uint32_t)(zz + u) * zstep) : f32x4v{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int u = 0; u < 16; ++u)
-                if (zz + u < S) add(wz[r][zz + u], v[u]);
+        if (G == 1) {
+            float* op = out + ((size_t)t * n_head + kvh * n_rep + r) * HD + d;
+            op[0] = __fdiv_rn(num.x, l_all[r]);
+            op[1] = __fdiv_rn(num.y, l_all[r]);
+            op[2] = __fdiv_rn(num.z, l_all[r]);
+            op[3] = __fdiv_rn(num.w, l_all[r]);
+        } else {
+            *(f32x4v*)&wpart[gi][4 * oo] = num;
         }
-        float* op = out + ((size_t)t * n_head + kvh * n_rep + r) * HD + d;
-        op[0] = __fdiv_rn(num.x, lsum[r]);
-        op[1] = __fdiv_rn(num.y, lsum[r]);
-        op[2] = __fdiv_rn(num.z, lsum[r]);
-        op[3] = __fdiv_rn(num.w, lsum[r]);
+    }
+    if (G == 1) return;
+    __syncthreads();
+    for (int o = threadIdx.x; o < n_rep * HD; o += kThreads) {
+        float v = wpart[0][o];
+        for (int gi = 1; gi < G; ++gi) v += wpart[gi][o];
+        const int r = o / HD, d = o - r * HD;
+        out[((size_t)t * n_head + kvh * n_rep + r) * HD + d] = __fdiv_rn(v, l_all[r]);
     }
 }
 
@@ -392,7 +477,7 @@ __global__ __launch_bounds__(kThreads) void k_attention(
 int attention_splits(int rows, int pos0, int n_kv) {
     const int L_max = pos0 + rows;
     const int64_t base = (int64_t)n_kv * rows;
-    int S = (int)std::min<int64_t>(std::max<int64_t>(1, (1024 + base - 1) / base),
+    int S = (int)std::min<int64_t>(std::max<int64_t>(1, (512 + base - 1) / base),
                                    (L_max + kChunk - 1) / kChunk);
     S = std::min(S, kMaxSplits);
     if ((int64_t)rows * n_kv > kAttnCounters) S = 1;
@@ -411,9 +496,20 @@ hipError_t launch_attention_hd(const float* q, const float* kc, const float* vc,
     const int split_len = ((L_max + S - 1) / S + kChunk - 1) / kChunk * kChunk;
     S = (L_max + split_len - 1) / split_len;
     const float scale = 1.0f / std::sqrt((float)HD);  // engine.cpp:121, IEEE on the host
-    hipLaunchKernelGGL((k_attention<HD>), dim3((unsigned)n_kv, (unsigned)rows, (unsigned)S),
-                       dim3(kThreads), 0, stream, q, kc, vc, n_head, n_kv, pos0, split_len, scale,
-                       part, counters, out, rope_base, k_new);
+    const int n_rep = n_head / n_kv;
+#define CLLM_ATTENTION(R)                                                                        \
+    hipLaunchKernelGGL((k_attention<HD, R>), dim3((unsigned)n_kv, (unsigned)rows, (unsigned)S),   \
+                       dim3(kThreads), 0, stream, q, kc, vc, n_head, n_kv, pos0, split_len, scale, part, counters,   \
+                       out, rope_base, k_new)
+    if (n_rep == 1)
+        CLLM_ATTENTION(1);
+    else if (n_rep == 2)
+        CLLM_ATTENTION(2);
+    else if (n_rep <= 4)
+        CLLM_ATTENTION(4);
+    else
+        CLLM_ATTENTION(8);
+#undef CLLM_ATTENTION
     return hipGetLastError();
 }
 
@@ -737,13 +833,15 @@ int attention_mfma_groups(int rows, int n_head, int n_kv, int head_dim) {
 
 // Many query rows go to the MFMA kernel (no workspace, no sequence split); with fewer than 32
 // of its workgroups (under 49 rows at 8 KV heads of 4 query heads each) the split kernel,
-// which spreads each row's positions over the device, is as fast or faster (MI355X, head_dim
-// 128: 32 rows at pos0 1024 89.9 us split / 94.5 MFMA, 64 rows 168 / 97).
+// which spreads each row's positions over the device, is faster (MI355X, head_dim 128, us, split
+// against MFMA kernel: 32 rows of 32 + 8 heads at the end of 1024 positions 24 / 92, of 4096 67 /
+// 338), and so it is up to 32 rows of any heads (32 + 32 heads at 1024: 1 row 11 / 49, 32 rows
+// 41 / 51).
 bool attention_uses_mfma(int rows, int pos0, int n_head, int n_kv, int head_dim) {
     const int kind = tuning().attention_kind.load();
     if (kind != 0) return kind == 2;
     (void)pos0;
-    return attention_mfma_groups(rows, n_head, n_kv, head_dim) >= 32;
+    return rows > 32 && attention_mfma_groups(rows, n_head, n_kv, head_dim) >= 32;
 }
 
 void attention_plan_name(int rows, int pos0, int n_head, int n_kv, int head_dim, char* buf,
