@@ -25,10 +25,12 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 
 #include "device_utils.h"
 #include "launch.h"
+#include "mfma_common.h"
 
 namespace cllm_hip {
 
@@ -572,19 +574,34 @@ __device__ __forceinline__ float quad_reduce(float x) {
     return MAX ? fmaxf(b0, b1) : b0 + b1;
 }
 
+// LDS of a workgroup: the partial outputs, maxima and sums of the parts; while the steps run, the
+// split queries lie where the partial outputs of the first waves come later.
 template <int HD, int CT, int W>
-__global__ __launch_bounds__(W * 64) void k_attention_mfma(
-    const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc,
-    int n_head, int n_kv, int rows, int pos0, int n_blocks, float scale, float* __restrict__ out) {
-    constexpr int COLS = 16 * CT;
+struct AttnLds {
+    static constexpr int COLS = 16 * CT, NS = W + 1, PAD = HD + 4;
+    float o[NS][COLS][PAD];
+    float m[NS][COLS], l[NS][COLS];
+    float den[2][COLS];
+    int slot_blk[NS];  // the block (0 or 1) whose partial a slot holds, -1: none
+};
+
+// One pass over a workgroup's two row blocks; true where an output of this thread is not finite.
+template <int HD, int CT, int W, bool SPLIT>
+__device__ __forceinline__ bool attention_pass(
+    AttnLds<HD, CT, W>& sm, const float* __restrict__ q, const float* __restrict__ kc,
+    const float* __restrict__ vc, int n_head, int n_kv, int rows, int pos0, int n_blocks, float scale,
+    float* __restrict__ out) {
+    using Lds = AttnLds<HD, CT, W>;
+    constexpr int COLS = Lds::COLS;
     constexpr int DQ = HD / 4;   // K and Q values per lane and row
     constexpr int DV = HD / 16;  // V values per lane and row
-    constexpr int PAD = HD + 4;  // LDS row stride of the partial outputs
-    constexpr int NS = W + 1;    // partial slots: one per wave, one more for the straddling wave
-    __shared__ float o_sm[NS][COLS][PAD];
-    __shared__ float m_sm[NS][COLS], l_sm[NS][COLS];
-    __shared__ float den_sm[2][COLS];
-    __shared__ int slot_blk[NS];  // the block (0 or 1) whose partial a slot holds, -1: none
+    constexpr int NS = Lds::NS;  // partial slots: one per wave, one more for the straddling wave
+    constexpr int SP = SPLIT ? 32 : 16;  // positions per step
+    auto& o_sm = sm.o;
+    auto& m_sm = sm.m;
+    auto& l_sm = sm.l;
+    auto& den_sm = sm.den;
+    auto& slot_blk = sm.slot_blk;
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -598,7 +615,7 @@ __global__ __launch_bounds__(W * 64) void k_attention_mfma(
     const int blk_row[2] = {pair * rpb, (n_blocks - 1 - pair) * rpb};
     const bool two = n_blocks - 1 - pair > pair;
     const int len[2] = {pos0 + min(rows, blk_row[0] + rpb), two ? pos0 + min(rows, blk_row[1] + rpb) : 0};
-    const int nA = (len[0] + 15) / 16, T = nA + (len[1] + 15) / 16;
+    const int nA = (len[0] + SP - 1) / SP, T = nA + (len[1] + SP - 1) / SP;
     const int g0 = wave * T / W, g1 = (wave + 1) * T / W;
     if (lane == 0) {
         slot_blk[wave] = g0 >= g1 ? -1 : g1 > nA ? 1 : 0;
@@ -609,12 +626,54 @@ __global__ __launch_bounds__(W * 64) void k_attention_mfma(
         }
     }
 
+    // SPLIT: the columns of both blocks as three bf16 parts, [block][part][column][HD], 16-byte
+    // chunk c of a column at slot c ^ (column & 7)
+    uint8_t* qlds = (uint8_t*)sm.o;
+    constexpr int QCOL = HD * 2, QPART = COLS * QCOL;
+    static_assert(!SPLIT || 6 * QPART <= W * COLS * Lds::PAD * 4, "the queries end below the straddling wave's slot");
+    if constexpr (SPLIT) {
+        for (int i = threadIdx.x; i < 2 * COLS * (HD / 8); i += W * 64) {
+            const int blk = i / (COLS * (HD / 8)), c = (i / (HD / 8)) % COLS, ch = i % (HD / 8);
+            const int t = blk_row[blk] + c / n_rep;
+            const bool valid = c < used && t < rows;  // unused columns: zeros
+            const float* qr = q + ((size_t)min(t, rows - 1) * n_head + g * n_rep + c % n_rep) * HD + 8 * ch;
+            const f32x4 v0 = *(const f32x4*)qr, v1 = *(const f32x4*)(qr + 4);
+            float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = valid ? v[e] : 0.0f;
+            wbf8 p[3];
+            split8<3>(v, p);
+#pragma unroll
+            for (int u = 0; u < 3; ++u)
+                *(wbf8*)(qlds + (blk * 3 + u) * QPART + c * QCOL + ((ch ^ (c & 7)) << 4)) = p[u];
+        }
+        __syncthreads();
+    }
+
+    f32x4 o[CT][DV];
+    float m_run[CT], l_run[CT];
+    // a part's partial: result register r of dim tile dt is dim DV (4 (l / 16) + r) + dt of
+    // column l % 16, so each lane stores HD / 4 consecutive dims
+    auto store_partial = [&](int slot) {
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            const int c = ct * 16 + col16;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int dt = 0; dt < DV; ++dt) o_sm[slot][c][DV * (4 * quad + r) + dt] = o[ct][dt][r];
+            if (quad == 0) {
+                m_sm[slot][c] = m_run[ct];
+                l_sm[slot][c] = l_run[ct];
+            }
+        }
+    };
+
     for (int part = 0; part < 2; ++part) {
         const int s0 = part == 0 ? g0 : max(g0, nA) - nA;
         const int s1 = part == 0 ? min(g1, nA) : g1 - nA;
         if (s0 >= s1) continue;
         const int r0 = blk_row[part], L = len[part];
-        const int slot = part == 0 && g1 > nA ? W : wave;
 
         // the queries of this lane's columns (unused columns: zeros from a row in bounds);
         // lim = the last position a column sees (-1: an unused column, every score masked)
@@ -626,6 +685,7 @@ __global__ __launch_bounds__(W * 64) void k_attention_mfma(
             const int t = r0 + c / n_rep;
             const bool valid = c < used && t < rows;
             lim[ct] = valid ? pos0 + t : -1;
+            if constexpr (SPLIT) continue;
             const float* qr = q + ((size_t)min(t, rows - 1) * n_head + g * n_rep + c % n_rep) * HD + DQ * quad;
 #pragma unroll
             for (int j = 0; j < DQ; j += 4) {
@@ -636,8 +696,6 @@ __global__ __launch_bounds__(W * 64) void k_attention_mfma(
                 qf[ct][j + 3] = valid ? v.w : 0.0f;
             }
         }
-        f32x4 o[CT][DV];
-        float m_run[CT], l_run[CT];
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
             m_run[ct] = -INFINITY;
@@ -646,6 +704,127 @@ __global__ __launch_bounds__(W * 64) void k_attention_mfma(
             for (int dt = 0; dt < DV; ++dt) o[ct][dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         }
 
+        if constexpr (SPLIT) {
+            // K rows 32 s + 16 u + l % 16 (dims 32 ks + 8 (l / 16) + e), V rows 32 s + 4 (l / 16) +
+            // i and 16 more (dims DV (l % 16) + d), positions and steps clamped as below
+            constexpr int KS = HD / 32, VH = DV / 4;
+            float kf[2][8 * KS], vf[VH][8][4];
+            auto load_k = [&](int s, int u) {
+                const float* kr = kc + (size_t)g * HD + 8 * quad +
+                                  (size_t)min(min(s, s1 - 1) * 32 + 16 * u + col16, L - 1) * kv_dim;
+#pragma unroll
+                for (int j = 0; j < 2 * KS; ++j) {
+                    const f32x4 v = *(const f32x4*)(kr + 32 * (j >> 1) + 4 * (j & 1));
+                    kf[u][4 * j] = v.x; kf[u][4 * j + 1] = v.y; kf[u][4 * j + 2] = v.z; kf[u][4 * j + 3] = v.w;
+                }
+            };
+            auto load_v = [&](int s, int hf) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int p = min(s, s1 - 1) * 32 + (e < 4 ? 0 : 16) + 4 * quad + (e & 3);
+                    const f32x4 v = *(const f32x4*)(vg + (size_t)min(p, L - 1) * kv_dim + 4 * hf);
+                    vf[hf][e][0] = v.x; vf[hf][e][1] = v.y; vf[hf][e][2] = v.z; vf[hf][e][3] = v.w;
+                }
+            };
+            const uint8_t* qb = qlds + part * 3 * QPART + col16 * QCOL;
+            load_k(s0, 0);
+            load_k(s0, 1);
+            for (int s = s0; s < s1; ++s) {
+                // the scores, transposed: 16 positions x 16 columns per (u, ct). Loads go out half
+                // a step ahead of their use, in the registers the phase before has left.
+                f32x4 sc[2][CT];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (u < VH) load_v(s, u);
+                    f32x4 hi[CT], lo[CT];
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) hi[ct] = lo[ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int ks = 0; ks < KS; ++ks) {
+                        wbf8 kp[3];
+                        split8<3>(&kf[u][8 * ks], kp);
+#pragma unroll
+                        for (int ct = 0; ct < CT; ++ct) {
+                            const uint8_t* p = qb + ct * 16 * QCOL + (((4 * ks + quad) ^ (col16 & 7)) << 4);
+                            const wbf8 q0 = *(const wbf8*)p, q1 = *(const wbf8*)(p + QPART);
+                            const wbf8 q2 = *(const wbf8*)(p + 2 * QPART);
+                            lo[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[2], q0, lo[ct], 0, 0, 0);
+                            hi[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[0], q0, hi[ct], 0, 0, 0);
+                            lo[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[0], q2, lo[ct], 0, 0, 0);
+                            lo[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[1], q1, lo[ct], 0, 0, 0);
+                            lo[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[1], q0, lo[ct], 0, 0, 0);
+                            lo[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[0], q1, lo[ct], 0, 0, 0);
+                        }
+                    }
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) sc[u][ct] = hi[ct] + lo[ct];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                // the online softmax of the step's 32 positions, as below
+                wbf8 pp[CT][3];
+                float cr[CT];
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) {
+                    float sv[8], pr[8], mx = -INFINITY;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const int p = s * 32 + (e < 4 ? 0 : 16) + 4 * quad + (e & 3);
+                        sv[e] = p <= lim[ct] ? __fmul_rn(sc[e >> 2][ct][e & 3], scale) : -INFINITY;
+                        mx = fmaxf(mx, sv[e]);
+                    }
+                    mx = quad_reduce<true>(mx);
+                    const float mo = m_run[ct], mn = fmaxf(mo, mx);
+                    float ps = 0.0f;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float x = expf(sv[e] - mn);
+                        pr[e] = sv[e] == -INFINITY ? 0.0f : x;
+                        ps += pr[e];
+                    }
+                    ps = quad_reduce<false>(ps);
+                    const float x = expf(mo - mn);
+                    cr[ct] = mo == -INFINITY ? 0.0f : x;
+                    m_run[ct] = mn;
+                    l_run[ct] = __builtin_fmaf(l_run[ct], cr[ct], ps);
+                    split8<3>(pr, pp[ct]);
+                }
+                // P.V of 32 positions per dim tile, small products first, then into the output
+#pragma unroll
+                for (int hf = 0; hf < VH; ++hf) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    load_k(s + 1, hf);
+                    if (VH == 1) load_k(s + 1, 1);
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) {
+                        float v[8];
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) v[e] = vf[hf][e][d];
+                        wbf8 vp[3];
+                        split8<3>(v, vp);
+                        f32x4 t[CT];
+                        const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                        for (int ct = 0; ct < CT; ++ct) t[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[2], pp[ct][0], zero, 0, 0, 0);
+#pragma unroll
+                        for (int ct = 0; ct < CT; ++ct) t[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[0], pp[ct][2], t[ct], 0, 0, 0);
+#pragma unroll
+                        for (int ct = 0; ct < CT; ++ct) t[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[1], pp[ct][1], t[ct], 0, 0, 0);
+#pragma unroll
+                        for (int ct = 0; ct < CT; ++ct) t[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[1], pp[ct][0], t[ct], 0, 0, 0);
+#pragma unroll
+                        for (int ct = 0; ct < CT; ++ct) t[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[0], pp[ct][1], t[ct], 0, 0, 0);
+#pragma unroll
+                        for (int ct = 0; ct < CT; ++ct) t[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[0], pp[ct][0], t[ct], 0, 0, 0);
+#pragma unroll
+                        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r)
+                                o[ct][4 * hf + d][r] = __builtin_fmaf(o[ct][4 * hf + d][r], cr[ct], t[ct][r]);
+                    }
+                }
+            }
+        } else {
         // K row 16 s + l % 16 and V rows 16 s + 4 (l / 16) + i of step s, positions clamped
         // to the block's last (their scores are masked) and steps to the part's last
         float kf[DQ], vf[4][DV];
@@ -741,22 +920,13 @@ __global__ __launch_bounds__(W * 64) void k_attention_mfma(
         }
         softmax(s1 - 1, sa);
         pv();
-
-        // the part's partial: result register r of dim tile dt is dim DV (4 (l / 16) + r) + dt
-        // of column l % 16, so each lane stores HD / 4 consecutive dims
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-            const int c = ct * 16 + col16;
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int dt = 0; dt < DV; ++dt) o_sm[slot][c][DV * (4 * quad + r) + dt] = o[ct][dt][r];
-            if (quad == 0) {
-                m_sm[slot][c] = m_run[ct];
-                l_sm[slot][c] = l_run[ct];
-            }
         }
+        // the straddling wave's first part goes to its slot now; the others' wait until the
+        // queries are read no more
+        if (part == 0 && g1 > nA) store_partial(W);
     }
+    __syncthreads();
+    if (g0 < g1) store_partial(wave);
     __syncthreads();
     // per (block, column): the partials' weights e^(m - M) in place of their maxima, and the sum
     if (threadIdx.x < 2 * COLS) {
@@ -776,6 +946,7 @@ __global__ __launch_bounds__(W * 64) void k_attention_mfma(
         den_sm[blk][c] = den;
     }
     __syncthreads();
+    bool bad = false;
     for (int o4 = threadIdx.x; o4 < 2 * COLS * (HD / 4); o4 += W * 64) {
         const int blk = o4 / (COLS * (HD / 4));
         const int c = (o4 / (HD / 4)) % COLS, d = (o4 % (HD / 4)) * 4;
@@ -792,13 +963,30 @@ __global__ __launch_bounds__(W * 64) void k_attention_mfma(
             num.w = __builtin_fmaf(wgt, v.w, num.w);
         }
         const float den = den_sm[blk][c];
+        const f32x4 res = f32x4{__fdiv_rn(num.x, den), __fdiv_rn(num.y, den), __fdiv_rn(num.z, den), __fdiv_rn(num.w, den)};
+        bad |= !(fabsf(res.x) < INFINITY && fabsf(res.y) < INFINITY && fabsf(res.z) < INFINITY && fabsf(res.w) < INFINITY);
         float* orow = out + ((size_t)t * n_head + g * n_rep + c % n_rep) * HD + d;
-        orow[0] = __fdiv_rn(num.x, den);  // out is 4-byte aligned only
-        orow[1] = __fdiv_rn(num.y, den);
-        orow[2] = __fdiv_rn(num.z, den);
-        orow[3] = __fdiv_rn(num.w, den);
+        orow[0] = res.x;  // out is 4-byte aligned only
+        orow[1] = res.y;
+        orow[2] = res.z;
+        orow[3] = res.w;
     }
+    return bad;
 }
+
+template <int HD, int CT, int W>
+__global__ __launch_bounds__(W * 64) void k_attention_mfma(
+    const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc,
+    int n_head, int n_kv, int rows, int pos0, int n_blocks, float scale, float* __restrict__ out) {
+    extern __shared__ __align__(16) uint8_t attn_lds[];
+    auto& sm = *(AttnLds<HD, CT, W>*)attn_lds;
+    if constexpr (HD <= 128) {
+        const bool bad = attention_pass<HD, CT, W, true>(sm, q, kc, vc, n_head, n_kv, rows, pos0, n_blocks, scale, out);
+        if (!__syncthreads_or(bad)) return;
+    }
+    attention_pass<HD, CT, W, false>(sm, q, kc, vc, n_head, n_kv, rows, pos0, n_blocks, scale, out);
+}
+
 
 template <int HD, int CT, int W>
 hipError_t launch_attention_mfma_hd(const float* q, const float* kc, const float* vc, int rows,
@@ -807,8 +995,17 @@ hipError_t launch_attention_mfma_hd(const float* q, const float* kc, const float
     const int n_blocks = (rows + rpb - 1) / rpb;
     const int pairs = (n_blocks + 1) / 2;
     const float scale = 1.0f / std::sqrt((float)HD);  // engine.cpp:121, IEEE on the host
+    constexpr int LDS = sizeof(AttnLds<HD, CT, W>);
+    static_assert(LDS <= 160 * 1024, "LDS budget");
+    static std::atomic<bool> attr_set{false};
+    if (!attr_set.load(std::memory_order_acquire)) {
+        const hipError_t e = hipFuncSetAttribute((const void*)k_attention_mfma<HD, CT, W>,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+        if (e != hipSuccess) return e;
+        attr_set.store(true, std::memory_order_release);
+    }
     hipLaunchKernelGGL((k_attention_mfma<HD, CT, W>), dim3((unsigned)(n_kv * pairs)), dim3(W * 64),
-                       0, stream, q, kc, vc, n_head, n_kv, rows, pos0, n_blocks, scale, out);
+                       LDS, stream, q, kc, vc, n_head, n_kv, rows, pos0, n_blocks, scale, out);
     return hipGetLastError();
 }
 

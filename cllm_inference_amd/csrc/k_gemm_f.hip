@@ -108,30 +108,6 @@ template <> struct GUnit<T_Q3_K> {
     }
 };
 
-// P bf16 parts of eight fp32 values, largest first, each the rest rounded to nearest (two
-// values to a conversion).
-template <int P>
-__device__ __forceinline__ void split8(const float* v, wbf8 (&p)[P]) {
-    typedef float f32x2 __attribute__((ext_vector_type(2)));
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    uint32_t o[P][4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        float r0 = v[2 * e], r1 = v[2 * e + 1];
-#pragma unroll
-        for (int i = 0; i < P; ++i) {
-            const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{r0, r1}, bf16x2));
-            o[i][e] = u;
-            if (i + 1 < P) {
-                r0 -= __builtin_bit_cast(float, u << 16);
-                r1 -= __builtin_bit_cast(float, u & 0xFFFF0000u);
-            }
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < P; ++i) p[i] = __builtin_bit_cast(wbf8, wu4{o[i][0], o[i][1], o[i][2], o[i][3]});
-}
-
 template <uint32_t T, int WN, int WK, int MT>
 struct CfgF {
     static constexpr int THREADS = 64 * WN * WK;
