@@ -528,8 +528,22 @@ hipError_t launch_attention_hd(const float* q, const float* kc, const float* vc,
 
 // ------------------------------------------------------------- many query rows on MFMA
 
-// Prefill attention on the fp32 matrix cores (v_mfma_f32_16x16x4f32: the same fp32 products
-// and sums as the split kernel's FMAs, in another order).
+// Prefill attention with fp32's precision: at head_dim 64 and 128 on bf16 MFMA with split operands
+// (k_attention_mfma), at head_dim 256 and over caches of 4 GiB and up on the fp32 matrix cores
+// (k_attention_mfma_f32, v_mfma_f32_16x16x4f32).
+//
+// Split operands. K, V, the queries and the probabilities are sums of three bf16 parts (26 bits);
+// the six largest of the nine part products leave out less than an fp32 product's rounding, and
+// run 2.7 times as fast as the fp32 MFMA. The scores add the leading products apart from the
+// others (8 rounded additions at head_dim 128, where the fp32 form makes 32), and the P.V products
+// of 32 positions add up from zero, small ones first, before they join the output. Error against
+// 64 bits at 512 rows after 1024 positions (32 + 8 heads of 128): 2.0e-7, the fp32 form's 4.0e-7.
+// Queries are split once into LDS; each wave splits its own K and V rows, beside the MFMAs of the
+// rows before. What bounds it: that VALU work (about 1200 operations beside 192 MFMAs per 32
+// positions and 32 columns) and the loads' way, at two waves per SIMD. MI355X, us, fp32 form against
+// this one: 512 rows after 1024 positions 134.7 / 91, 300 rows 28.7 / 24; 200 rows of 16 + 16
+// heads of 64 13.3 / 12.3. A workgroup with an output that is not finite runs the fp32 form over its blocks (inf * 0
+// appears among the parts where fp32 has inf).
 //
 // Columns. A query block is COLS = 16 * CT (row, head) pairs of one KV head: column c is
 // query head c % n_rep of row r0 + c / n_rep, so the n_rep heads of a row and several rows
@@ -544,7 +558,8 @@ hipError_t launch_attention_hd(const float* q, const float* kc, const float* vc,
 // its K and V rows in that XCD's L2 when n_kv is 8. Two waves per SIMD (W = 8 up to head_dim
 // 128).
 //
-// One step, per 16-column tile: the scores come out transposed, S^T (16 positions x 16
+// One step of the fp32 form, per 16-column tile (the split form: two such score tiles, then P.V
+// over their 32 positions): the scores come out transposed, S^T (16 positions x 16
 // columns) = K Q^T over HD / 4 MFMAs (lane l holds K row l % 16 and Q column l % 16 at
 // dims (HD / 4) (l / 16) + j for MFMA j; even and odd j in two accumulators added at the end,
 // which halves the longest rounding chain), so lane l holds column l % 16's scores of
@@ -555,7 +570,7 @@ hipError_t launch_attention_hd(const float* q, const float* kc, const float* vc,
 // sum live in the four lanes l % 16 of its tile, reduced with v_permlane32_swap and
 // v_permlane16_swap (lanes l ^ 32, l ^ 16).
 //
-// Pipeline. A wave issues the next step's score MFMAs interleaved with this step's softmax
+// Pipeline (fp32 form). A wave issues the next step's score MFMAs interleaved with this step's softmax
 // (an MFMA every few VALU instructions, so the matrix pipe stays busy through the softmax),
 // then this step's P.V MFMAs; K rows are requested two steps ahead and V rows one step
 // ahead. Loads past a part's last step are clamped to rows in bounds instead of branched, so
@@ -586,17 +601,16 @@ struct AttnLds {
 };
 
 // One pass over a workgroup's two row blocks; true where an output of this thread is not finite.
-template <int HD, int CT, int W, bool SPLIT>
+template <int HD, int CT, int W>
 __device__ __forceinline__ bool attention_pass(
     AttnLds<HD, CT, W>& sm, const float* __restrict__ q, const float* __restrict__ kc,
     const float* __restrict__ vc, int n_head, int n_kv, int rows, int pos0, int n_blocks, float scale,
     float* __restrict__ out) {
     using Lds = AttnLds<HD, CT, W>;
     constexpr int COLS = Lds::COLS;
-    constexpr int DQ = HD / 4;   // K and Q values per lane and row
     constexpr int DV = HD / 16;  // V values per lane and row
     constexpr int NS = Lds::NS;  // partial slots: one per wave, one more for the straddling wave
-    constexpr int SP = SPLIT ? 32 : 16;  // positions per step
+    constexpr int SP = 32;       // positions per step
     auto& o_sm = sm.o;
     auto& m_sm = sm.m;
     auto& l_sm = sm.l;
@@ -609,8 +623,6 @@ __device__ __forceinline__ bool attention_pass(
     const int g = blockIdx.x % n_kv, pair = blockIdx.x / n_kv;
     const int n_rep = n_head / n_kv, rpb = COLS / n_rep, used = rpb * n_rep;
     const size_t kv_dim = (size_t)n_kv * HD;
-    const float* kg = kc + (size_t)g * HD + DQ * quad;
-    const float* vg = vc + (size_t)g * HD + DV * col16;
 
     const int blk_row[2] = {pair * rpb, (n_blocks - 1 - pair) * rpb};
     const bool two = n_blocks - 1 - pair > pair;
@@ -626,12 +638,12 @@ __device__ __forceinline__ bool attention_pass(
         }
     }
 
-    // SPLIT: the columns of both blocks as three bf16 parts, [block][part][column][HD], 16-byte
+    // the columns of both blocks as three bf16 parts, [block][part][column][HD], 16-byte
     // chunk c of a column at slot c ^ (column & 7)
     uint8_t* qlds = (uint8_t*)sm.o;
     constexpr int QCOL = HD * 2, QPART = COLS * QCOL;
-    static_assert(!SPLIT || 6 * QPART <= W * COLS * Lds::PAD * 4, "the queries end below the straddling wave's slot");
-    if constexpr (SPLIT) {
+    static_assert(6 * QPART <= W * COLS * Lds::PAD * 4, "the queries end below the straddling wave's slot");
+    {
         for (int i = threadIdx.x; i < 2 * COLS * (HD / 8); i += W * 64) {
             const int blk = i / (COLS * (HD / 8)), c = (i / (HD / 8)) % COLS, ch = i % (HD / 8);
             const int t = blk_row[blk] + c / n_rep;
@@ -650,11 +662,9 @@ __device__ __forceinline__ bool attention_pass(
         __syncthreads();
     }
 
-    f32x4 o[CT][DV];
-    float m_run[CT], l_run[CT];
     // a part's partial: result register r of dim tile dt is dim DV (4 (l / 16) + r) + dt of
     // column l % 16, so each lane stores HD / 4 consecutive dims
-    auto store_partial = [&](int slot) {
+    auto store_partial = [&](int slot, const f32x4 (&o)[CT][DV], const float (&m_run)[CT], const float (&l_run)[CT]) {
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
             const int c = ct * 16 + col16;
@@ -669,11 +679,321 @@ __device__ __forceinline__ bool attention_pass(
         }
     };
 
+    // one wave's share of a block; false where it has none
+    auto run_part = [&](int part, f32x4 (&o)[CT][DV], float (&m_run)[CT], float (&l_run)[CT]) {
+        const int s0 = part == 0 ? g0 : max(g0, nA) - nA;
+        const int s1 = part == 0 ? min(g1, nA) : g1 - nA;
+        if (s0 >= s1) return false;
+        const int r0 = blk_row[part], L = len[part];
+
+        // the last position a column sees (-1: an unused column, every score masked)
+        int lim[CT];
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            const int c = ct * 16 + col16, t = r0 + c / n_rep;
+            lim[ct] = c < used && t < rows ? pos0 + t : -1;
+        }
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            m_run[ct] = -INFINITY;
+            l_run[ct] = 0.0f;
+#pragma unroll
+            for (int dt = 0; dt < DV; ++dt) o[ct][dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+
+        // K rows 32 s + 16 u + l % 16 (dims 32 ks + 8 (l / 16) + e), V rows 32 s + 4 (l / 16) +
+        // i and 16 more (dims DV (l % 16) + d), positions and steps clamped as below
+        constexpr int KS = HD / 32, VH = DV / 4;
+        float kf[2][8 * KS], vf[VH][8][4];
+        // byte offsets of 32 bits (the host takes the fp32 pass for caches of 4 GiB and up)
+        const uint32_t row4 = 4u * (uint32_t)kv_dim;
+        const uint32_t k_at = 4u * (uint32_t)(g * HD + 8 * quad), v_at = 4u * (uint32_t)(g * HD + DV * col16);
+        auto load_k = [&](int s, int u) {
+            const uint32_t at = (uint32_t)min(min(s, s1 - 1) * 32 + 16 * u + col16, L - 1) * row4 + k_at;
+#pragma unroll
+            for (int j = 0; j < 2 * KS; ++j) {
+                const f32x4 v = *(const f32x4*)((const char*)kc + at + (128 * (j >> 1) + 16 * (j & 1)));
+                kf[u][4 * j] = v.x; kf[u][4 * j + 1] = v.y; kf[u][4 * j + 2] = v.z; kf[u][4 * j + 3] = v.w;
+            }
+        };
+        auto load_v = [&](int s, int hf) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int p = min(s, s1 - 1) * 32 + (e < 4 ? 0 : 16) + 4 * quad + (e & 3);
+                const f32x4 v = *(const f32x4*)((const char*)vc + ((uint32_t)min(p, L - 1) * row4 + v_at) + 16 * hf);
+                vf[hf][e][0] = v.x; vf[hf][e][1] = v.y; vf[hf][e][2] = v.z; vf[hf][e][3] = v.w;
+            }
+        };
+        const uint8_t* qb = qlds + part * 3 * QPART + col16 * QCOL;
+        load_k(s0, 0);
+        for (int s = s0; s < s1; ++s) {
+            // the scores, transposed: 16 positions x 16 columns per (u, ct). Loads go out one
+            // phase (half of the scores, half of P.V) ahead of their use.
+            f32x4 sc[2][CT];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (u == 0)
+                    load_k(s, 1);
+                else
+                    load_v(s, 0);
+                f32x4 hi[CT], lo[CT];
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) hi[ct] = lo[ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                // the next K step is split beside this one's MFMAs
+                wbf8 kps[2][3];
+                split8<3>(&kf[u][0], kps[0]);
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (ks + 1 < KS) split8<3>(&kf[u][8 * (ks + 1)], kps[(ks + 1) & 1]);
+                    const wbf8 (&kp)[3] = kps[ks & 1];
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) {
+                        const uint8_t* p = qb + ct * 16 * QCOL + (((4 * ks + quad) ^ (col16 & 7)) << 4);
+                        const wbf8 q0 = *(const wbf8*)p, q1 = *(const wbf8*)(p + QPART);
+                        const wbf8 q2 = *(const wbf8*)(p + 2 * QPART);
+                        lo[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[2], q0, lo[ct], 0, 0, 0);
+                        hi[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[0], q0, hi[ct], 0, 0, 0);
+                        lo[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[0], q2, lo[ct], 0, 0, 0);
+                        lo[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[1], q1, lo[ct], 0, 0, 0);
+                        lo[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[1], q0, lo[ct], 0, 0, 0);
+                        lo[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[0], q1, lo[ct], 0, 0, 0);
+                    }
+                    __builtin_amdgcn_sched_group_barrier(0x100, 3 * CT, 0);
+#pragma unroll
+                    for (int i = 0; i < 6 * CT; ++i) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // an MFMA
+                        __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // VALU beside it
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) sc[u][ct] = hi[ct] + lo[ct];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            // the online softmax of the step's 32 positions, as below
+            wbf8 pp[CT][3];
+            float cr[CT];
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+                float sv[8], pr[8], mx = -INFINITY;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int p = s * 32 + (e < 4 ? 0 : 16) + 4 * quad + (e & 3);
+                    sv[e] = p <= lim[ct] ? __fmul_rn(sc[e >> 2][ct][e & 3], scale) : -INFINITY;
+                    mx = fmaxf(mx, sv[e]);
+                }
+                mx = quad_reduce<true>(mx);
+                const float mo = m_run[ct], mn = fmaxf(mo, mx);
+                float ps = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float x = expf(sv[e] - mn);
+                    pr[e] = sv[e] == -INFINITY ? 0.0f : x;
+                    ps += pr[e];
+                }
+                ps = quad_reduce<false>(ps);
+                const float x = expf(mo - mn);
+                cr[ct] = mo == -INFINITY ? 0.0f : x;
+                m_run[ct] = mn;
+                l_run[ct] = __builtin_fmaf(l_run[ct], cr[ct], ps);
+                split8<3>(pr, pp[ct]);
+            }
+            // P.V of 32 positions per dim tile, small products first, then into the output
+#pragma unroll
+            for (int hf = 0; hf < VH; ++hf) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (hf + 1 < VH)
+                    load_v(s, hf + 1);
+                else
+                    load_k(s + 1, 0);
+                wbf8 vps[2][3];
+                auto split_v = [&](int d, wbf8 (&p)[3]) {
+                    float v[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[e] = vf[hf][e][d];
+                    split8<3>(v, p);
+                };
+                split_v(0, vps[0]);
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (d + 1 < 4) split_v(d + 1, vps[(d + 1) & 1]);
+                    const wbf8 (&vp)[3] = vps[d & 1];
+                    f32x4 t[CT];
+                    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) t[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[2], pp[ct][0], zero, 0, 0, 0);
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) t[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[0], pp[ct][2], t[ct], 0, 0, 0);
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) t[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[1], pp[ct][1], t[ct], 0, 0, 0);
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) t[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[1], pp[ct][0], t[ct], 0, 0, 0);
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) t[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[0], pp[ct][1], t[ct], 0, 0, 0);
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) t[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[0], pp[ct][0], t[ct], 0, 0, 0);
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            o[ct][4 * hf + d][r] = __builtin_fmaf(o[ct][4 * hf + d][r], cr[ct], t[ct][r]);
+#pragma unroll
+                    for (int i = 0; i < 6 * CT; ++i) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+                    }
+                }
+            }
+        }
+        return true;
+    };
+    // the straddling wave's first part goes to its slot at once; the others wait until the queries
+    // are read no more
+    f32x4 o[CT][DV];
+    float m_run[CT], l_run[CT];
+    for (int part = 0; part < 2; ++part)
+        if (run_part(part, o, m_run, l_run) && part == 0 && g1 > nA) store_partial(W, o, m_run, l_run);
+    __syncthreads();
+    if (g0 < g1) store_partial(wave, o, m_run, l_run);
+    __syncthreads();
+    // per (block, column): the partials' weights e^(m - M) in place of their maxima, and the sum
+    if (threadIdx.x < 2 * COLS) {
+        const int blk = threadIdx.x / COLS, c = threadIdx.x % COLS;
+        float M = -INFINITY;
+        for (int z = 0; z < NS; ++z)
+            if (slot_blk[z] == blk) M = fmaxf(M, m_sm[z][c]);
+        float den = 0.0f;
+        for (int z = 0; z < NS; ++z) {
+            if (slot_blk[z] != blk) continue;
+            const float m = m_sm[z][c];
+            const float e = expf(m - M);
+            const float wgt = m == -INFINITY ? 0.0f : e;
+            den = __builtin_fmaf(wgt, l_sm[z][c], den);
+            m_sm[z][c] = wgt;
+        }
+        den_sm[blk][c] = den;
+    }
+    __syncthreads();
+    bool bad = false;
+    for (int o4 = threadIdx.x; o4 < 2 * COLS * (HD / 4); o4 += W * 64) {
+        const int blk = o4 / (COLS * (HD / 4));
+        const int c = (o4 / (HD / 4)) % COLS, d = (o4 % (HD / 4)) * 4;
+        const int t = blk_row[blk] + c / n_rep;
+        if ((blk == 1 && !two) || c >= used || t >= rows) continue;
+        f32x4 num = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int z = 0; z < NS; ++z) {
+            if (slot_blk[z] != blk) continue;
+            const float wgt = m_sm[z][c];
+            const f32x4 v = *(const f32x4*)&o_sm[z][c][d];
+            num.x = __builtin_fmaf(wgt, v.x, num.x);
+            num.y = __builtin_fmaf(wgt, v.y, num.y);
+            num.z = __builtin_fmaf(wgt, v.z, num.z);
+            num.w = __builtin_fmaf(wgt, v.w, num.w);
+        }
+        const float den = den_sm[blk][c];
+        const f32x4 res = f32x4{__fdiv_rn(num.x, den), __fdiv_rn(num.y, den), __fdiv_rn(num.z, den), __fdiv_rn(num.w, den)};
+        bad |= !(fabsf(res.x) < INFINITY && fabsf(res.y) < INFINITY && fabsf(res.z) < INFINITY && fabsf(res.w) < INFINITY);
+        float* orow = out + ((size_t)t * n_head + g * n_rep + c % n_rep) * HD + d;
+        orow[0] = res.x;  // out is 4-byte aligned only
+        orow[1] = res.y;
+        orow[2] = res.z;
+        orow[3] = res.w;
+    }
+    return bad;
+}
+
+// One column in fp32, a wave's lanes over the dims, a position at a time: the rows whose split
+// products are not finite (inf * 0 appears among the parts where fp32 has inf).
+template <int HD>
+__device__ __noinline__ void attention_column(const float* qr, const float* kr, const float* vr,
+                                              size_t kv_dim, int L, float scale, float* orow) {
+    constexpr int E = HD / 64;
+    const int lane = threadIdx.x & 63;
+    float o[E], m = -INFINITY, l = 0.0f;
+#pragma unroll
+    for (int e = 0; e < E; ++e) o[e] = 0.0f;
+    for (int p = 0; p < L; ++p) {
+        float d = 0.0f;
+#pragma unroll
+        for (int e = 0; e < E; ++e) d = __builtin_fmaf(qr[lane + 64 * e], kr[p * kv_dim + lane + 64 * e], d);
+#pragma unroll
+        for (int i = 32; i >= 1; i >>= 1) d += __shfl_xor(d, i, 64);
+        const float s = __fmul_rn(d, scale), mn = fmaxf(m, s);
+        const float pr = s == -INFINITY ? 0.0f : expf(s - mn), cr = m == -INFINITY ? 0.0f : expf(m - mn);
+        l = __builtin_fmaf(l, cr, pr);
+#pragma unroll
+        for (int e = 0; e < E; ++e) o[e] = __builtin_fmaf(pr, vr[p * kv_dim + lane + 64 * e], o[e] * cr);
+        m = mn;
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) orow[lane + 64 * e] = __fdiv_rn(o[e], l);
+}
+
+template <int HD, int CT, int W>
+__global__ __launch_bounds__(W * 64) void k_attention_mfma(
+    const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc,
+    int n_head, int n_kv, int rows, int pos0, int n_blocks, float scale, float* __restrict__ out) {
+    extern __shared__ __align__(16) uint8_t attn_lds[];
+    auto& sm = *(AttnLds<HD, CT, W>*)attn_lds;
+    const bool bad = attention_pass<HD, CT, W>(sm, q, kc, vc, n_head, n_kv, rows, pos0, n_blocks, scale, out);
+    if (!__syncthreads_or(bad)) return;
+    const int g = blockIdx.x % n_kv, pair = blockIdx.x / n_kv, n_rep = n_head / n_kv, rpb = 16 * CT / n_rep;
+    for (int i = threadIdx.x >> 6; i < 2 * rpb * n_rep; i += W) {
+        const int blk = i / (rpb * n_rep), c = i % (rpb * n_rep), b = blk ? n_blocks - 1 - pair : pair;
+        const int t = b * rpb + c / n_rep;
+        if ((blk == 1 && b <= pair) || t >= rows) continue;
+        const size_t at = ((size_t)t * n_head + g * n_rep + c % n_rep) * HD;
+        attention_column<HD>(q + at, kc + (size_t)g * HD, vc + (size_t)g * HD, (size_t)n_kv * HD, pos0 + t + 1,
+                             scale, out + at);
+    }
+}
+
+template <int HD, int CT, int W>
+__global__ __launch_bounds__(W * 64) void k_attention_mfma_f32(
+    const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc,
+    int n_head, int n_kv, int rows, int pos0, int n_blocks, float scale, float* __restrict__ out) {
+    constexpr int COLS = 16 * CT;
+    constexpr int DQ = HD / 4;   // K and Q values per lane and row
+    constexpr int DV = HD / 16;  // V values per lane and row
+    constexpr int PAD = HD + 4;  // LDS row stride of the partial outputs
+    constexpr int NS = W + 1;    // partial slots: one per wave, one more for the straddling wave
+    __shared__ float o_sm[NS][COLS][PAD];
+    __shared__ float m_sm[NS][COLS], l_sm[NS][COLS];
+    __shared__ float den_sm[2][COLS];
+    __shared__ int slot_blk[NS];  // the block (0 or 1) whose partial a slot holds, -1: none
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col16 = lane & 15, quad = lane >> 4;
+    const int g = blockIdx.x % n_kv, pair = blockIdx.x / n_kv;
+    const int n_rep = n_head / n_kv, rpb = COLS / n_rep, used = rpb * n_rep;
+    const size_t kv_dim = (size_t)n_kv * HD;
+    const float* kg = kc + (size_t)g * HD + DQ * quad;
+    const float* vg = vc + (size_t)g * HD + DV * col16;
+
+    const int blk_row[2] = {pair * rpb, (n_blocks - 1 - pair) * rpb};
+    const bool two = n_blocks - 1 - pair > pair;
+    const int len[2] = {pos0 + min(rows, blk_row[0] + rpb), two ? pos0 + min(rows, blk_row[1] + rpb) : 0};
+    const int nA = (len[0] + 15) / 16, T = nA + (len[1] + 15) / 16;
+    const int g0 = wave * T / W, g1 = (wave + 1) * T / W;
+    if (lane == 0) {
+        slot_blk[wave] = g0 >= g1 ? -1 : g1 > nA ? 1 : 0;
+        if (wave == 0) {
+            bool straddle = false;
+            for (int w = 0; w < W; ++w) straddle |= w * T / W < nA && nA < (w + 1) * T / W;
+            slot_blk[W] = straddle ? 0 : -1;
+        }
+    }
+
     for (int part = 0; part < 2; ++part) {
         const int s0 = part == 0 ? g0 : max(g0, nA) - nA;
         const int s1 = part == 0 ? min(g1, nA) : g1 - nA;
         if (s0 >= s1) continue;
         const int r0 = blk_row[part], L = len[part];
+        const int slot = part == 0 && g1 > nA ? W : wave;
 
         // the queries of this lane's columns (unused columns: zeros from a row in bounds);
         // lim = the last position a column sees (-1: an unused column, every score masked)
@@ -685,7 +1005,6 @@ __device__ __forceinline__ bool attention_pass(
             const int t = r0 + c / n_rep;
             const bool valid = c < used && t < rows;
             lim[ct] = valid ? pos0 + t : -1;
-            if constexpr (SPLIT) continue;
             const float* qr = q + ((size_t)min(t, rows - 1) * n_head + g * n_rep + c % n_rep) * HD + DQ * quad;
 #pragma unroll
             for (int j = 0; j < DQ; j += 4) {
@@ -696,6 +1015,8 @@ __device__ __forceinline__ bool attention_pass(
                 qf[ct][j + 3] = valid ? v.w : 0.0f;
             }
         }
+        f32x4 o[CT][DV];
+        float m_run[CT], l_run[CT];
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
             m_run[ct] = -INFINITY;
@@ -704,127 +1025,6 @@ __device__ __forceinline__ bool attention_pass(
             for (int dt = 0; dt < DV; ++dt) o[ct][dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         }
 
-        if constexpr (SPLIT) {
-            // K rows 32 s + 16 u + l % 16 (dims 32 ks + 8 (l / 16) + e), V rows 32 s + 4 (l / 16) +
-            // i and 16 more (dims DV (l % 16) + d), positions and steps clamped as below
-            constexpr int KS = HD / 32, VH = DV / 4;
-            float kf[2][8 * KS], vf[VH][8][4];
-            auto load_k = [&](int s, int u) {
-                const float* kr = kc + (size_t)g * HD + 8 * quad +
-                                  (size_t)min(min(s, s1 - 1) * 32 + 16 * u + col16, L - 1) * kv_dim;
-#pragma unroll
-                for (int j = 0; j < 2 * KS; ++j) {
-                    const f32x4 v = *(const f32x4*)(kr + 32 * (j >> 1) + 4 * (j & 1));
-                    kf[u][4 * j] = v.x; kf[u][4 * j + 1] = v.y; kf[u][4 * j + 2] = v.z; kf[u][4 * j + 3] = v.w;
-                }
-            };
-            auto load_v = [&](int s, int hf) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int p = min(s, s1 - 1) * 32 + (e < 4 ? 0 : 16) + 4 * quad + (e & 3);
-                    const f32x4 v = *(const f32x4*)(vg + (size_t)min(p, L - 1) * kv_dim + 4 * hf);
-                    vf[hf][e][0] = v.x; vf[hf][e][1] = v.y; vf[hf][e][2] = v.z; vf[hf][e][3] = v.w;
-                }
-            };
-            const uint8_t* qb = qlds + part * 3 * QPART + col16 * QCOL;
-            load_k(s0, 0);
-            load_k(s0, 1);
-            for (int s = s0; s < s1; ++s) {
-                // the scores, transposed: 16 positions x 16 columns per (u, ct). Loads go out half
-                // a step ahead of their use, in the registers the phase before has left.
-                f32x4 sc[2][CT];
-#pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (u < VH) load_v(s, u);
-                    f32x4 hi[CT], lo[CT];
-#pragma unroll
-                    for (int ct = 0; ct < CT; ++ct) hi[ct] = lo[ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                    for (int ks = 0; ks < KS; ++ks) {
-                        wbf8 kp[3];
-                        split8<3>(&kf[u][8 * ks], kp);
-#pragma unroll
-                        for (int ct = 0; ct < CT; ++ct) {
-                            const uint8_t* p = qb + ct * 16 * QCOL + (((4 * ks + quad) ^ (col16 & 7)) << 4);
-                            const wbf8 q0 = *(const wbf8*)p, q1 = *(const wbf8*)(p + QPART);
-                            const wbf8 q2 = *(const wbf8*)(p + 2 * QPART);
-                            lo[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[2], q0, lo[ct], 0, 0, 0);
-                            hi[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[0], q0, hi[ct], 0, 0, 0);
-                            lo[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[0], q2, lo[ct], 0, 0, 0);
-                            lo[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[1], q1, lo[ct], 0, 0, 0);
-                            lo[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[1], q0, lo[ct], 0, 0, 0);
-                            lo[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[0], q1, lo[ct], 0, 0, 0);
-                        }
-                    }
-#pragma unroll
-                    for (int ct = 0; ct < CT; ++ct) sc[u][ct] = hi[ct] + lo[ct];
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                // the online softmax of the step's 32 positions, as below
-                wbf8 pp[CT][3];
-                float cr[CT];
-#pragma unroll
-                for (int ct = 0; ct < CT; ++ct) {
-                    float sv[8], pr[8], mx = -INFINITY;
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const int p = s * 32 + (e < 4 ? 0 : 16) + 4 * quad + (e & 3);
-                        sv[e] = p <= lim[ct] ? __fmul_rn(sc[e >> 2][ct][e & 3], scale) : -INFINITY;
-                        mx = fmaxf(mx, sv[e]);
-                    }
-                    mx = quad_reduce<true>(mx);
-                    const float mo = m_run[ct], mn = fmaxf(mo, mx);
-                    float ps = 0.0f;
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const float x = expf(sv[e] - mn);
-                        pr[e] = sv[e] == -INFINITY ? 0.0f : x;
-                        ps += pr[e];
-                    }
-                    ps = quad_reduce<false>(ps);
-                    const float x = expf(mo - mn);
-                    cr[ct] = mo == -INFINITY ? 0.0f : x;
-                    m_run[ct] = mn;
-                    l_run[ct] = __builtin_fmaf(l_run[ct], cr[ct], ps);
-                    split8<3>(pr, pp[ct]);
-                }
-                // P.V of 32 positions per dim tile, small products first, then into the output
-#pragma unroll
-                for (int hf = 0; hf < VH; ++hf) {
-                    __builtin_amdgcn_sched_barrier(0);
-                    load_k(s + 1, hf);
-                    if (VH == 1) load_k(s + 1, 1);
-#pragma unroll
-                    for (int d = 0; d < 4; ++d) {
-                        float v[8];
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) v[e] = vf[hf][e][d];
-                        wbf8 vp[3];
-                        split8<3>(v, vp);
-                        f32x4 t[CT];
-                        const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                        for (int ct = 0; ct < CT; ++ct) t[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[2], pp[ct][0], zero, 0, 0, 0);
-#pragma unroll
-                        for (int ct = 0; ct < CT; ++ct) t[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[0], pp[ct][2], t[ct], 0, 0, 0);
-#pragma unroll
-                        for (int ct = 0; ct < CT; ++ct) t[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[1], pp[ct][1], t[ct], 0, 0, 0);
-#pragma unroll
-                        for (int ct = 0; ct < CT; ++ct) t[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[1], pp[ct][0], t[ct], 0, 0, 0);
-#pragma unroll
-                        for (int ct = 0; ct < CT; ++ct) t[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[0], pp[ct][1], t[ct], 0, 0, 0);
-#pragma unroll
-                        for (int ct = 0; ct < CT; ++ct) t[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[0], pp[ct][0], t[ct], 0, 0, 0);
-#pragma unroll
-                        for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-                            for (int r = 0; r < 4; ++r)
-                                o[ct][4 * hf + d][r] = __builtin_fmaf(o[ct][4 * hf + d][r], cr[ct], t[ct][r]);
-                    }
-                }
-            }
-        } else {
         // K row 16 s + l % 16 and V rows 16 s + 4 (l / 16) + i of step s, positions clamped
         // to the block's last (their scores are masked) and steps to the part's last
         float kf[DQ], vf[4][DV];
@@ -920,13 +1120,22 @@ __device__ __forceinline__ bool attention_pass(
         }
         softmax(s1 - 1, sa);
         pv();
+
+        // the part's partial: result register r of dim tile dt is dim DV (4 (l / 16) + r) + dt
+        // of column l % 16, so each lane stores HD / 4 consecutive dims
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            const int c = ct * 16 + col16;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int dt = 0; dt < DV; ++dt) o_sm[slot][c][DV * (4 * quad + r) + dt] = o[ct][dt][r];
+            if (quad == 0) {
+                m_sm[slot][c] = m_run[ct];
+                l_sm[slot][c] = l_run[ct];
+            }
         }
-        // the straddling wave's first part goes to its slot now; the others' wait until the
-        // queries are read no more
-        if (part == 0 && g1 > nA) store_partial(W);
     }
-    __syncthreads();
-    if (g0 < g1) store_partial(wave);
     __syncthreads();
     // per (block, column): the partials' weights e^(m - M) in place of their maxima, and the sum
     if (threadIdx.x < 2 * COLS) {
@@ -946,7 +1155,6 @@ __device__ __forceinline__ bool attention_pass(
         den_sm[blk][c] = den;
     }
     __syncthreads();
-    bool bad = false;
     for (int o4 = threadIdx.x; o4 < 2 * COLS * (HD / 4); o4 += W * 64) {
         const int blk = o4 / (COLS * (HD / 4));
         const int c = (o4 / (HD / 4)) % COLS, d = (o4 % (HD / 4)) * 4;
@@ -963,30 +1171,13 @@ __device__ __forceinline__ bool attention_pass(
             num.w = __builtin_fmaf(wgt, v.w, num.w);
         }
         const float den = den_sm[blk][c];
-        const f32x4 res = f32x4{__fdiv_rn(num.x, den), __fdiv_rn(num.y, den), __fdiv_rn(num.z, den), __fdiv_rn(num.w, den)};
-        bad |= !(fabsf(res.x) < INFINITY && fabsf(res.y) < INFINITY && fabsf(res.z) < INFINITY && fabsf(res.w) < INFINITY);
         float* orow = out + ((size_t)t * n_head + g * n_rep + c % n_rep) * HD + d;
-        orow[0] = res.x;  // out is 4-byte aligned only
-        orow[1] = res.y;
-        orow[2] = res.z;
-        orow[3] = res.w;
+        orow[0] = __fdiv_rn(num.x, den);  // out is 4-byte aligned only
+        orow[1] = __fdiv_rn(num.y, den);
+        orow[2] = __fdiv_rn(num.z, den);
+        orow[3] = __fdiv_rn(num.w, den);
     }
-    return bad;
 }
-
-template <int HD, int CT, int W>
-__global__ __launch_bounds__(W * 64) void k_attention_mfma(
-    const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc,
-    int n_head, int n_kv, int rows, int pos0, int n_blocks, float scale, float* __restrict__ out) {
-    extern __shared__ __align__(16) uint8_t attn_lds[];
-    auto& sm = *(AttnLds<HD, CT, W>*)attn_lds;
-    if constexpr (HD <= 128) {
-        const bool bad = attention_pass<HD, CT, W, true>(sm, q, kc, vc, n_head, n_kv, rows, pos0, n_blocks, scale, out);
-        if (!__syncthreads_or(bad)) return;
-    }
-    attention_pass<HD, CT, W, false>(sm, q, kc, vc, n_head, n_kv, rows, pos0, n_blocks, scale, out);
-}
-
 
 template <int HD, int CT, int W>
 hipError_t launch_attention_mfma_hd(const float* q, const float* kc, const float* vc, int rows,
@@ -995,17 +1186,26 @@ hipError_t launch_attention_mfma_hd(const float* q, const float* kc, const float
     const int n_blocks = (rows + rpb - 1) / rpb;
     const int pairs = (n_blocks + 1) / 2;
     const float scale = 1.0f / std::sqrt((float)HD);  // engine.cpp:121, IEEE on the host
-    constexpr int LDS = sizeof(AttnLds<HD, CT, W>);
-    static_assert(LDS <= 160 * 1024, "LDS budget");
-    static std::atomic<bool> attr_set{false};
-    if (!attr_set.load(std::memory_order_acquire)) {
-        const hipError_t e = hipFuncSetAttribute((const void*)k_attention_mfma<HD, CT, W>,
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-        if (e != hipSuccess) return e;
-        attr_set.store(true, std::memory_order_release);
+    const dim3 grid((unsigned)(n_kv * pairs));
+    if constexpr (HD <= 128) {
+        // (the split form's offsets into the caches have 32 bits)
+        if ((uint64_t)(pos0 + rows) * (uint64_t)(n_kv * HD) * sizeof(float) < (1ull << 32)) {
+            constexpr int LDS = sizeof(AttnLds<HD, CT, W>);
+            static_assert(LDS <= 160 * 1024 - 1024, "LDS budget");
+            static std::atomic<bool> attr_set{false};
+            if (!attr_set.load(std::memory_order_acquire)) {
+                const hipError_t e = hipFuncSetAttribute((const void*)k_attention_mfma<HD, CT, W>,
+                                                         hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+                if (e != hipSuccess) return e;
+                attr_set.store(true, std::memory_order_release);
+            }
+            hipLaunchKernelGGL((k_attention_mfma<HD, CT, W>), grid, dim3(W * 64), LDS, stream, q, kc, vc,
+                               n_head, n_kv, rows, pos0, n_blocks, scale, out);
+            return hipGetLastError();
+        }
     }
-    hipLaunchKernelGGL((k_attention_mfma<HD, CT, W>), dim3((unsigned)(n_kv * pairs)), dim3(W * 64),
-                       LDS, stream, q, kc, vc, n_head, n_kv, rows, pos0, n_blocks, scale, out);
+    hipLaunchKernelGGL((k_attention_mfma_f32<HD, CT, W>), grid, dim3(W * 64), 0, stream, q, kc, vc, n_head,
+                       n_kv, rows, pos0, n_blocks, scale, out);
     return hipGetLastError();
 }
 
@@ -1050,6 +1250,9 @@ bool attention_uses_mfma(int rows, int pos0, int n_head, int n_kv, int head_dim)
     const int kind = tuning().attention_kind.load();
     if (kind != 0) return kind == 2;
     (void)pos0;
+    // one or two heads per KV head: 128 rows of 16 + 8 heads of 128 after 1024 positions 51 / 69,
+    // 128 rows of 8 + 4 heads of 256 55 / 110, 256 rows 102 / 109
+    if (n_head / n_kv <= 2 && rows <= (head_dim == 256 ? 256 : 128)) return false;
     return rows > 32 && attention_mfma_groups(rows, n_head, n_kv, head_dim) >= 32;
 }
 
