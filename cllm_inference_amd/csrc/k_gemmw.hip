@@ -22,6 +22,7 @@
 // the raw Q4_K bytes of the half (header + 64 quant bytes per row), dx, the activations as
 // fp16 integers (16-byte chunks swizzled by token, so the fragment reads of 16 consecutive
 // tokens fall on distinct banks) and dx * bsum split into bf16 parts.
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 
@@ -909,7 +910,7 @@ __device__ __forceinline__ uint32_t bits_to_byte_bit4(uint32_t x) {
     return ((x | (x << 7) | (x << 14) | (x << 21)) & 0x01010101u) << 4;
 }
 
-template <uint32_t T, int W, int MT, bool ANY>
+template <uint32_t T, int W, int MT, bool ANY, bool COMP>
 __global__ __launch_bounds__(64 * W) void k_gemmw_b32(const uint8_t* __restrict__ w,
                                                       uint32_t row_bytes, int k, int n, int m,
                                                       const _Float16* __restrict__ qh,
@@ -1000,11 +1001,11 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_b32(const uint8_t* __restrict_
         }
     };
 
-    wf16 yacc[MT];
+    wf16 yacc[MT], part2[COMP ? MT : 1];  // part2: the sum of two stages
 #pragma unroll
     for (int a = 0; a < MT; ++a)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) yacc[a][r] = 0.0f;
+        for (int r = 0; r < 16; ++r) yacc[a][r] = part2[COMP ? a : 0][r] = 0.0f;
 
     float* scratch = (float*)(lds + 2 * C::STAGE) + wave * 128;
     const int wrow = wave * 32 + r32;
@@ -1103,10 +1104,30 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_b32(const uint8_t* __restrict_
                 const int b = it / MT, mt = it % MT;
                 const float dx = dxv[it % 3];
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    yacc[mt][r] = fmaf(dx, dr[b][r] * f[it & 1][r], yacc[mt][r]);
-                asm volatile("" : "+v"(yacc[mt]));  // not sunk past the stage's branches
+                for (int r = 0; r < 16; ++r) {
+                    const float i = dr[b][r] * f[it & 1][r];
+                    if constexpr (COMP)
+                        part2[mt][r] = fmaf(dx, i, part2[mt][r]);
+                    else
+                        yacc[mt][r] = fmaf(dx, i, yacc[mt][r]);
+                }
+                if constexpr (COMP)  // not sunk past the stage's branches
+                    asm volatile("" : "+v"(part2[mt]));
+                else
+                    asm volatile("" : "+v"(yacc[mt]));
             });
+        if constexpr (COMP) {
+            if (((s - s_begin) & 1) || s + 1 == s_end) {
+#pragma unroll
+                for (int a = 0; a < MT; ++a)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const float t = yacc[a][r] + part2[a][r];
+                        part2[a][r] = (yacc[a][r] - t) + part2[a][r];
+                        yacc[a][r] = t;
+                    }
+            }
+        }
         if (more) wait_vm();
         __syncthreads();
         if (more) patch(s + 1, nxt);
@@ -1257,6 +1278,9 @@ Plan plan_for(uint32_t type, int k, int n, int m) {
         }
         p.splits = best;
     }
+    // (the splits' sums are added one after the other: with 8, K = 8224 was further off the
+    // 64-bit result than the GEMV)
+    if (k % 256 != 0) p.splits = std::min(p.splits, 4);
     const int sp = tu.gemm_splits.load(std::memory_order_relaxed);
     if (sp >= 1 && sp <= 16 && sp <= k / kKS) p.splits = sp;
     return p;
@@ -1309,14 +1333,14 @@ hipError_t launch_q6(const uint8_t* w, int k, int n, int m, const _Float16* qh, 
     return hipGetLastError();
 }
 
-template <uint32_t T, int W, int MT, bool ANY>
+template <uint32_t T, int W, int MT, bool ANY, bool COMP>
 hipError_t launch_b32(const uint8_t* w, int k, int n, int m, const _Float16* qh, const float* xs,
                       const float* bias, float* y, float* part, int* counters, int splits,
                       hipStream_t stream) {
     using C = CfgB<T, W, MT, ANY>;
     static bool attr_set = false;
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void*)k_gemmw_b32<T, W, MT, ANY>,
+        hipError_t e = hipFuncSetAttribute((const void*)k_gemmw_b32<T, W, MT, ANY, COMP>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
         if (e != hipSuccess) return e;
         attr_set = true;
@@ -1325,7 +1349,7 @@ hipError_t launch_b32(const uint8_t* w, int k, int n, int m, const _Float16* qh,
     const int tiles = ((n + C::BN - 1) / C::BN) * ((m + C::BM - 1) / C::BM);
     const int stages = (k + kKS - 1) / kKS;
     const int per = k % 256 == 0 ? 2 * ((stages / 2 + splits - 1) / splits) : (stages + splits - 1) / splits;
-    hipLaunchKernelGGL((k_gemmw_b32<T, W, MT, ANY>), dim3((unsigned)tiles, (unsigned)splits),
+    hipLaunchKernelGGL((k_gemmw_b32<T, W, MT, ANY, COMP>), dim3((unsigned)tiles, (unsigned)splits),
                        dim3(C::THREADS), C::LDS, stream, w, row_bytes, k, n, m, qh, xs, bias, y, part,
                        counters, per);
     return hipGetLastError();
@@ -1421,13 +1445,17 @@ hipError_t gemmw_dispatch(uint32_t type, const Segs& sg, int k, int m, const flo
 #define CLLM_GEMMW_B32(TT)                                                                    \
         if (type == TT) {                                                                      \
             if (k % kKS != 0 && p.mt == 2)                                                     \
-                e = launch_b32<TT, 4, 2, true>(w, k, n, m, qh, xs, bias, y, part, counters, p.splits, stream); \
+                e = launch_b32<TT, 4, 2, true, true>(w, k, n, m, qh, xs, bias, y, part, counters, p.splits, stream); \
             else if (k % kKS != 0)                                                             \
-                e = launch_b32<TT, 4, 1, true>(w, k, n, m, qh, xs, bias, y, part, counters, p.splits, stream); \
+                e = launch_b32<TT, 4, 1, true, true>(w, k, n, m, qh, xs, bias, y, part, counters, p.splits, stream); \
+            else if (k % 256 != 0 && p.mt == 2)                                                \
+                e = launch_b32<TT, 4, 2, false, true>(w, k, n, m, qh, xs, bias, y, part, counters, p.splits, stream); \
+            else if (k % 256 != 0)                                                             \
+                e = launch_b32<TT, 4, 1, false, true>(w, k, n, m, qh, xs, bias, y, part, counters, p.splits, stream); \
             else if (p.mt == 2)                                                                \
-                e = launch_b32<TT, 4, 2, false>(w, k, n, m, qh, xs, bias, y, part, counters, p.splits, stream); \
+                e = launch_b32<TT, 4, 2, false, false>(w, k, n, m, qh, xs, bias, y, part, counters, p.splits, stream); \
             else                                                                               \
-                e = launch_b32<TT, 4, 1, false>(w, k, n, m, qh, xs, bias, y, part, counters, p.splits, stream); \
+                e = launch_b32<TT, 4, 1, false, false>(w, k, n, m, qh, xs, bias, y, part, counters, p.splits, stream); \
         }
         CLLM_GEMMW_B32(T_Q8_0)
         CLLM_GEMMW_B32(T_Q4_0)
