@@ -9,8 +9,10 @@
 //     out_h = sum_t (e_t / sum) v_t; decode (495) and prefill (581-583, query t of the
 //     batch sees pos0 + t + 1 positions).
 //
-// Two attention kernels: k_attention (below; decode, and a few rows over a long cache) and
-// k_attention_mfma (many query rows, on fp32 MFMA; its layout is described above it).
+// Three attention kernels: k_attention (below; decode, and a few rows over a long cache),
+// k_attention_mfma (many query rows at head_dim 64 and 128, on bf16 MFMA with fp32 operands split
+// in three) and k_attention_mfma_f32 (many query rows at head_dim 256, or over caches of 4 GiB and
+// more, on fp32 MFMA); the layouts of the latter two are described above them.
 //
 // Attention layout. One workgroup per (KV head, query row, sequence split); it serves the
 // n_rep query heads of that KV head, so every K and V row is loaded once for all of them. Its
@@ -74,7 +76,7 @@ __global__ __launch_bounds__(256) void k_rope_neox(float* __restrict__ x, int n_
 // ----------------------------------------------------------------------------- attention
 
 constexpr int kThreads = 256;
-constexpr int kChunk = 64;       // positions per online-softmax step
+constexpr int kChunk = 64;       // a sequence split is a multiple of this many positions
 constexpr int kLanesPerPos = 16; // lanes sharing one K row
 constexpr int kMaxRep = 8;       // query heads per KV head
 constexpr int kAttnCounters = 1024;  // (row, KV head) pairs a split launch may have

@@ -1252,8 +1252,9 @@ Plan plan_for(uint32_t type, int k, int n, int m) {
     const int tiles = ((n + bn - 1) / bn) * ((m + bm - 1) / bm);
     p.splits = choose_splits(tiles, k / kKS, target, min_stages);
     // Above 256 rows on 128 x 64 tiles, while the tiles make fewer than two rounds of the
-    // CUs' resident workgroups (1 per CU for the 32-element block types' tile at 306 VGPRs, 2
-    // for the K-quants'): the split count (1, 2 or 4) whose workgroups run in the fewest
+    // CUs' workgroup slots (taken as 1 per CU for the 32-element block types' tile, 2 for the
+    // K-quants'; the former's registers now allow 2 as well, the split counts stay as they were
+    // measured): the split count (1, 2 or 4) whose workgroups run in the fewest
     // stage-rounds,
     // ceil(workgroups / slots) x ceil(stages / splits); on a tie, more splits only while the CUs
     // are not yet filled. Measured at m = 384 .. 1024: on 4096 x 14336 and 4096 x 4096 this

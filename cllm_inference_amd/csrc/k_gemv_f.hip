@@ -1,5 +1,5 @@
 // k_gemv_f.hip -- float-dot GEMV for the weight types without a vec_dot kernel: F32, F16,
-// Q4_1, Q5_1, Q8_1, Q2_K and Q3_K.
+// Q4_1, Q5_1, Q8_1, Q2_K and Q3_K (larger batches take k_gemm_f.hip, with the same decoders).
 //
 // The reference routes these through the fallback of matmul_quant (src/core/quant.cpp:
 // 1404-1430; matmul_quant_batch runs it row by row, 1471-1474): each weight row is
