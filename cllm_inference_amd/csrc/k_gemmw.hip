@@ -1122,8 +1122,10 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_b32(const uint8_t* __restrict_
                 for (int a = 0; a < MT; ++a)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
+                        // (an infinite sum has no rounding to carry: inf - inf would be NaN)
                         const float t = yacc[a][r] + part2[a][r];
-                        part2[a][r] = (yacc[a][r] - t) + part2[a][r];
+                        const float c = (yacc[a][r] - t) + part2[a][r];
+                        part2[a][r] = fabsf(t) < INFINITY ? c : 0.0f;
                         yacc[a][r] = t;
                     }
             }

@@ -66,3 +66,39 @@ def test_rows_of_whole_blocks_under_capture(gpu, orc):
         check_close(y.cpu().numpy(), yo, exact, abs_sum, f"replay {rep}")
         again = gpu.matmul_quant_dev(xd, wd, qt, None, k, n)
         assert torch.equal(again, eager)
+
+
+BLOCK_BYTES = {S.Q8_0: 34, S.Q4_0: 18, S.Q5_0: 22}
+
+
+@pytest.mark.parametrize("splits", [0, 2])
+@pytest.mark.parametrize("k", [896, 1120])
+@pytest.mark.parametrize("qt", [S.Q8_0, S.Q4_0, S.Q5_0])
+def test_rows_of_whole_blocks_infinite_sums(gpu, orc, qt, k, splits):
+    """A weight block whose scale is infinite, in an early, a middle and the last stage, makes its
+    row's outputs the infinities (or, with an opposite one or a zero block sum, the NaNs) that the
+    fp32 sums of the oracle give; the other rows keep the bits they have without it."""
+    n, m, nb = 70, 40, k // 32
+    w = S.make_weight(qt, n, k, 3)
+    x = S.make_activation(m, k, 4)
+    bad = w.copy()
+    blocks = bad.reshape(n, nb, BLOCK_BYTES[qt])
+    for row, blk, bits in ((1, 0, 0x7C00), (7, 0, 0xFC00), (33, 9, 0x7C00), (34, nb - 1, 0x7C00),
+                           (50, 5, 0x7E00)):
+        blocks[row, blk, :2] = np.frombuffer(np.uint16(bits).tobytes(), np.uint8)
+    # two opposite infinities
+    for blk, bits in ((2, 0x7C00), (nb - 2, 0xFC00)):
+        blocks[60, blk, :2] = np.frombuffer(np.uint16(bits).tobytes(), np.uint8)
+    gpu.tune("gemm_splits", splits)
+    try:
+        assert gpu.matmul_route(qt, k, n, m) == "mfma"
+        got = gpu.matmul_quant_dev(_dev(x), _dev(bad), qt, None, k, n).cpu().numpy()
+        clean = gpu.matmul_quant_dev(_dev(x), _dev(w), qt, None, k, n).cpu().numpy()
+    finally:
+        gpu.tune("gemm_splits")
+    want = orc.matmul(x, bad, qt, None, k, n, m).reshape(m, n)
+    rows = [1, 7, 33, 34, 50, 60]
+    assert np.isinf(want[:, [1, 7, 33, 34]]).sum() > 3 * m  # the case holds what it is about
+    assert np.array_equal(got[:, rows], want[:, rows], equal_nan=True)
+    keep = [r for r in range(n) if r not in rows]
+    assert np.array_equal(got[:, keep], clean[:, keep])
