@@ -1093,7 +1093,8 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_b32(const uint8_t* __restrict_
                 const uint8_t* arow = act + tok * 256;
                 bf[it & 1][0] = *(const wh8*)(arow + (((4 * b + 2 * h) ^ sw) << 4));
                 bf[it & 1][1] = *(const wh8*)(arow + (((4 * b + 2 * h + 1) ^ sw) << 4));
-                dxv[it % 3] = dxl[tok * 4 + b];
+                // (past K: zero times what the clamped load left there, which may be infinite)
+                dxv[it % 3] = ANY && 4 * s + b >= nb ? 0.0f : dxl[tok * 4 + b];
             },
             [&](int it) {
                 const wf16 zero = {};

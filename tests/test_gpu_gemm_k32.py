@@ -102,3 +102,23 @@ def test_rows_of_whole_blocks_infinite_sums(gpu, orc, qt, k, splits):
     assert np.array_equal(got[:, rows], want[:, rows], equal_nan=True)
     keep = [r for r in range(n) if r not in rows]
     assert np.array_equal(got[:, keep], clean[:, keep])
+
+
+@pytest.mark.parametrize("qt", [S.Q8_0, S.Q4_0, S.Q5_0])
+def test_rows_of_whole_blocks_infinite_last_activation_scale(gpu, orc, qt):
+    """Pre-quantized rows whose last block has an infinite scale, at a K that ends inside a stage:
+    the blocks past K add nothing, so the outputs are the GEMV's infinities and NaNs."""
+    n, k, m = 40, 1120, 20
+    w = _dev(S.make_weight(qt, n, k, 5))
+    qs, sc, bs = gpu.quantize_q8_0_dev(_dev(S.make_activation(m, k, 6)))
+    sc[3, -1] = float("inf")
+    sc[4, 0] = float("inf")
+    assert gpu.matmul_route(qt, k, n, m) == "mfma"
+    got = gpu.gemv_q8_dev(w, qt, k, n, qs, sc, bs).cpu().numpy()
+    # at most 8 rows take the GEMV
+    want = np.concatenate([gpu.gemv_q8_dev(w, qt, k, n, qs[t:t + 4].clone(), sc[t:t + 4].clone(),
+                                           bs[t:t + 4].clone()).cpu().numpy() for t in range(0, m, 4)])
+    assert np.isinf(want[3:5]).any()
+    assert np.array_equal(got[3:5], want[3:5], equal_nan=True)
+    rest = [t for t in range(m) if t not in (3, 4)]
+    np.testing.assert_allclose(got[rest], want[rest], rtol=1e-4, atol=1e-5 * np.abs(want[rest]).max())
