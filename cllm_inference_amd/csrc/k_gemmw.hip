@@ -1011,14 +1011,19 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_b32(const uint8_t* __restrict_
     const int wrow = wave * 32 + r32;
     // ANY: the lead of this lane's row window, 0 or 2 bytes
     const uint32_t sh = ANY ? ((uint32_t)min(n0 + wrow, n - 1) * row_bytes) & 2u : 0u;
-    // ANY: the half dword at the end of the matrix (its row, n - 1, starts at a multiple of 4)
+    // ANY, before the last stage: the half dword at the end of the matrix (its row, n - 1, starts
+    // at a multiple of 4), and no activation scale for the blocks past K (the loads left the last
+    // block's there, and an infinite one times their zeros would be NaN)
     const bool half_dword = ANY && (w_bytes & 2u) && n0 + C::BN >= n;
     auto patch = [&](int s, uint8_t* st) {
-        if (!half_dword || s != stages - 1) return;
-        if (threadIdx.x == 0) {
+        if (!ANY || s != stages - 1 || (!half_dword && nb % 4 == 0)) return;
+        if (half_dword && threadIdx.x == 0) {
             const uint32_t at = w_bytes - 2u - ((uint32_t)(n - 1) * row_bytes + (uint32_t)s * (uint32_t)C::SROW);
             *(uint16_t*)(st + C::OFF_W + (n - 1 - n0) * C::LROW + at) = *(const uint16_t*)(w + w_bytes - 2u);
         }
+        static_assert(BM * 4 <= C::THREADS, "a thread per activation scale");
+        if (threadIdx.x < BM * 4 && 4 * s + (int)(threadIdx.x & 3) >= nb)
+            ((float*)(st + C::OFF_DX))[threadIdx.x] = 0.0f;
         __syncthreads();
     };
 
@@ -1093,8 +1098,7 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_b32(const uint8_t* __restrict_
                 const uint8_t* arow = act + tok * 256;
                 bf[it & 1][0] = *(const wh8*)(arow + (((4 * b + 2 * h) ^ sw) << 4));
                 bf[it & 1][1] = *(const wh8*)(arow + (((4 * b + 2 * h + 1) ^ sw) << 4));
-                // (past K: zero times what the clamped load left there, which may be infinite)
-                dxv[it % 3] = ANY && 4 * s + b >= nb ? 0.0f : dxl[tok * 4 + b];
+                dxv[it % 3] = dxl[tok * 4 + b];
             },
             [&](int it) {
                 const wf16 zero = {};
@@ -1123,10 +1127,11 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_b32(const uint8_t* __restrict_
                 for (int a = 0; a < MT; ++a)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
-                        // (an infinite sum has no rounding to carry: inf - inf would be NaN)
+                        // (taken off the sum held to finite values: an infinite sum carries on as
+                        // the infinity it is, where inf - inf would make it NaN)
                         const float t = yacc[a][r] + part2[a][r];
-                        const float c = (yacc[a][r] - t) + part2[a][r];
-                        part2[a][r] = fabsf(t) < INFINITY ? c : 0.0f;
+                        const float f = __builtin_amdgcn_fmed3f(t, -__FLT_MAX__, __FLT_MAX__);
+                        part2[a][r] = (yacc[a][r] - f) + part2[a][r];
                         yacc[a][r] = t;
                     }
             }
