@@ -25,6 +25,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
+#include <type_traits>
 
 #include "ggml_blocks.h"
 #include "launch.h"
@@ -94,7 +95,8 @@ struct Cfg {
 // Each wave waits for its slot stores to complete before the workgroup barrier, and the
 // counter is bumped after that barrier; the workgroup's LDS (free once every wave has left
 // its main loop) carries the verdict.
-template <int NI, int W, class Val, class Tok, class Row>
+// WIDE: these additions in 64 bits (4 splits of 7200 elements 7.7e-8 off the exact sum, now 7.1e-8).
+template <int NI, int W, bool WIDE = false, class Val, class Tok, class Row>
 __device__ __forceinline__ void store_tile(int n, int m, const float* __restrict__ bias,
                                            float* __restrict__ y, float* __restrict__ part,
                                            int* __restrict__ counters, uint8_t* lds, int wave,
@@ -149,7 +151,7 @@ __device__ __forceinline__ void store_tile(int n, int m, const float* __restrict
     }
     __syncthreads();
     if (!*last) return;
-    float acc[NI][16];
+    std::conditional_t<WIDE, double, float> acc[NI][16];
     for (int sp = 0; sp < splits; ++sp) {
         const bool own = sp == (int)blockIdx.y;
 #pragma unroll
@@ -171,7 +173,7 @@ __device__ __forceinline__ void store_tile(int n, int m, const float* __restrict
                 acc[i][2 * r2 + 1] = sp == 0 ? x1 : acc[i][2 * r2 + 1] + x1;
             }
     }
-    write_out([&](int i, int r) { return acc[i][r]; });
+    write_out([&](int i, int r) { return (float)acc[i][r]; });
 }
 
 // The MFMA work of N items (one block of weights against one token tile each), software
@@ -1149,7 +1151,7 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_b32(const uint8_t* __restrict_
         for (int s = s_begin; s < s_end; ++s) run_stage(s);
     }
 
-    store_tile<MT, W>(
+    store_tile<MT, W, COMP>(
         n, m, bias, y, part, counters, lds, wave, [&](int i, int r) { return yacc[i][r]; },
         [&](int i) { return m0 + i * 32 + r32; },
         [&](int i, int r) { return n0 + wave * 32 + 8 * (r >> 2) + 4 * h + (r & 3); });
@@ -1287,9 +1289,20 @@ Plan plan_for(uint32_t type, int k, int n, int m) {
         }
         p.splits = best;
     }
-    // (the splits' sums are added one after the other: with 8, K = 8224 was further off the
-    // 64-bit result than the GEMV)
-    if (k % 256 != 0) p.splits = std::min(p.splits, 4);
+    // Rows that are no multiple of 256 long: a wave's chain of stages is what a small matrix takes
+    // (1.6 us each, 2.2 on 64 tokens), against 4 to 6 us per launch of 8 rows on the GEMV, which
+    // was the faster of the two up to 40 rows and 8 M weights. So there a split goes down to 3
+    // stages while the workgroups do not outnumber the CUs, from 1024 elements (K = 896 is 15 us
+    // whole, GEMV 16).
+    // MI355X, us, at 8 stages per split / now / GEMV, Q8_0: 300 x 1184 at 17 rows 21.2 / 15.8 /
+    // 17.4, 512 x 3008 at 17 25.7 / 18.6 / 17.8, 1000 x 4000 at 17 31.6 / 21.7 / 21.1, at 33 42 /
+    // 29 / 36. Error against 64 bits, of 300 x 1184: 6.5e-8 / 7.1e-8 / 7.5e-8.
+    // 4 splits at most: with 8, K = 8224 was further off the 64-bit result than the GEMV.
+    if (k % 256 != 0) {
+        if (k >= 1024 && m <= 40 && (int64_t)n * k < (int64_t(8) << 20))
+            p.splits = std::max(p.splits, choose_splits(tiles, k / kKS, cus, 3));
+        p.splits = std::min(p.splits, 4);
+    }
     const int sp = tu.gemm_splits.load(std::memory_order_relaxed);
     if (sp >= 1 && sp <= 16 && sp <= k / kKS) p.splits = sp;
     return p;

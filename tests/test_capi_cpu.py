@@ -242,6 +242,19 @@ def _libc():
 PROT_READ, PROT_WRITE, MAP_SHARED, MAP_PRIVATE, MAP_FIXED = 1, 2, 1, 2, 0x10
 
 
+def test_plans_of_rows_no_multiple_of_256():
+    """Up to 40 rows over matrices of less than 8 M weights split K down to 3 stages of 128 elements
+    per split (at most 4 splits, no more workgroups than CUs); K below 1024, larger batches and
+    larger matrices keep 8 stages per split."""
+    def splits(k, n, m):
+        assert C.matmul_route(8, k, n, m) == "mfma"
+        return int(C.matmul_plan(8, k, n, m).split("splits=")[1])
+    assert splits(896, 300, 17) == 1
+    assert splits(1056, 300, 17) == 2 and splits(1184, 2000, 40) == 2 and splits(1184, 300, 41) == 1
+    assert splits(1568, 300, 24) == 4 and splits(4000, 1000, 17) == 4 and splits(4000, 1000, 41) == 2
+    assert splits(4000, 2048, 40) == 4 and splits(4000, 4096, 40) == 2 and splits(8224, 300, 100) == 4
+
+
 def test_attention_plans():
     """Many query rows take the MFMA kernel (32 or more of its workgroups: n_kv x pairs of
     row blocks of 32 / n_rep rows, 16 / n_rep at head_dim 256); fewer rows, and a decode row,
