@@ -1232,30 +1232,59 @@ size_t attention_workspace_bytes(int rows, int n_head, int head_dim) {
 
 namespace {
 
-// Workgroups of the MFMA kernel: n_kv x pairs of row blocks (16 CT columns per block).
-int attention_mfma_groups(int rows, int n_head, int n_kv, int head_dim) {
-    const int ct = head_dim == 256 ? 1 : 2;
-    const int rpb = 16 * ct / (n_head / n_kv);
-    const int n_blocks = (rows + rpb - 1) / rpb;
-    return n_kv * ((n_blocks + 1) / 2);
+// Row blocks of the MFMA kernel (16 CT columns, rpb whole rows each) and its workgroups: n_kv x
+// pairs of blocks.
+struct MfmaGrid {
+    int rpb, blocks, groups;
+};
+MfmaGrid attention_mfma_grid(int rows, int n_head, int n_kv, int head_dim) {
+    const int rpb = 16 * (head_dim == 256 ? 1 : 2) / (n_head / n_kv);
+    const int blocks = (rows + rpb - 1) / rpb;
+    return {rpb, blocks, n_kv * ((blocks + 1) / 2)};
 }
 
 }  // namespace
 
-// Many query rows go to the MFMA kernel (no workspace, no sequence split); with fewer than 32
-// of its workgroups (under 49 rows at 8 KV heads of 4 query heads each) the split kernel,
-// which spreads each row's positions over the device, is faster (MI355X, head_dim 128, us, split
-// against MFMA kernel: 32 rows of 32 + 8 heads at the end of 1024 positions 24 / 92, of 4096 67 /
-// 338), and so it is up to 32 rows of any heads (32 + 32 heads at 1024: 1 row 11 / 49, 32 rows
-// 41 / 51).
+// Which kernel: the split kernel's work grows with the rows (each reads its KV head's cache rows
+// anew, from L2), the MFMA kernel's time hardly does while its workgroups fit the CUs.
+//
+// From three query heads per KV head: the MFMA kernel (no workspace, no sequence split) from 33
+// rows where it has 32 workgroups (49 rows at 8 KV heads of 4 query heads). MI355X, head_dim 128,
+// us, split against MFMA kernel: 32 rows of 32 + 8 heads at the end of 1024 positions 24 / 69, of
+// 4096 67 / 220; 64 rows of 64 + 16 heads at 4096 229 / 223, of 128 + 32 heads at 1024 114 / 70.
+// Over up to 112 positions (head_dim 64 and 128) the MFMA kernel's waves have one step or none and
+// wait for its loads one after the other, so fewer rows stay on the split kernel: 96 rows of 32 + 8 heads 12.3 / 16.1,
+// 48 of 64 + 8 10.3 / 14.7, of 64 + 16 11.6 / 14.9 (80 rows 17.6 / 16.1); not 64 rows over 64
+// positions, two whole steps, which take 12.6 on either.
+//
+// One or two query heads per KV head, up to 128 rows (256 at head_dim 256; more take the MFMA
+// kernel): the faster by two measured rates. The split kernel reads rows x n_kv x positions K and
+// V rows at 32 TB/s, with about as much as 64 positions take for the ends of each workgroup; the
+// waves of an MFMA workgroup share the steps over its two blocks' positions and take 4.2 / 6.5 /
+// 3.0 us for one (32 positions at head_dim 64 and 128, 16 at 256). MI355X, us, split against MFMA kernel at 64 + 64 heads of 128: 32 rows after 4096
+// positions 364 / 117, 8 rows 90 / 117, 128 rows after 1024 368 / 71, 24 rows over 24 9 / 11; 16 + 16
+// heads of 64, 128 rows after 256 17 / 21, after 4096 160 / 138; 128 rows of 8 + 4 heads of 256
+// after 1024 55 / 103, of 32 + 32 319 / 115.
 bool attention_uses_mfma(int rows, int pos0, int n_head, int n_kv, int head_dim) {
     const int kind = tuning().attention_kind.load();
     if (kind != 0) return kind == 2;
-    (void)pos0;
-    // one or two heads per KV head: 128 rows of 16 + 8 heads of 128 after 1024 positions 51 / 69,
-    // 128 rows of 8 + 4 heads of 256 55 / 110, 256 rows 102 / 109
-    if (n_head / n_kv <= 2 && rows <= (head_dim == 256 ? 256 : 128)) return false;
-    return rows > 32 && attention_mfma_groups(rows, n_head, n_kv, head_dim) >= 32;
+    const int n_rep = n_head / n_kv;
+    const MfmaGrid g = attention_mfma_grid(rows, n_head, n_kv, head_dim);
+    const int positions = pos0 + rows;
+    if (n_rep > 2) {
+        const int few = head_dim == 256 ? 0 : n_rep <= 4 ? 960 : positions < 64 ? 512 : 0;
+        if (positions <= 112 && positions != 64 && rows * n_kv < few) return false;
+        return rows > 32 && g.groups >= 32;
+    }
+    if (rows > (head_dim == 256 ? 256 : 128)) return g.groups >= 32;
+    const float split_us = (float)rows * n_kv * (pos0 + 0.5f * rows + 64.0f) * (8.0f * head_dim) / 32e6f;
+    const int step = head_dim == 256 ? 16 : 32, waves = head_dim == 256 ? 4 : 8;
+    const float start_us = head_dim == 64 ? 0.0f : 2.0f;  // beyond the split kernel's
+    const float step_us = head_dim == 64 ? 4.2f : head_dim == 128 ? 6.5f : 3.0f;
+    const int steps = (pos0 + std::min(rows, g.rpb) + step - 1) / step +
+                      (g.blocks > 1 ? (positions + step - 1) / step : 0);
+    const int rounds = (g.groups + 255) / 256;
+    return split_us > start_us + step_us * (float)((steps + waves - 1) / waves * rounds);
 }
 
 void attention_plan_name(int rows, int pos0, int n_head, int n_kv, int head_dim, char* buf,
@@ -1263,7 +1292,7 @@ void attention_plan_name(int rows, int pos0, int n_head, int n_kv, int head_dim,
     if (attention_uses_mfma(rows, pos0, n_head, n_kv, head_dim)) {
         const int ct = head_dim == 256 ? 1 : 2, w = head_dim == 256 ? 4 : 8;
         snprintf(buf, cap, "k_attention_mfma<%d,%d,%d> workgroups=%d", head_dim, ct, w,
-                 attention_mfma_groups(rows, n_head, n_kv, head_dim));
+                 attention_mfma_grid(rows, n_head, n_kv, head_dim).groups);
     } else {
         snprintf(buf, cap, "k_attention<%d> splits=%d", head_dim, attention_splits(rows, pos0, n_kv));
     }

@@ -281,6 +281,23 @@ def test_attention_plans():
         C.tune("attention_kernel", 3)
 
 
+def test_attention_plans_by_cost():
+    """One or two query heads per KV head: the kernel by the work, whatever the row count says
+    (many KV heads over a long cache take the MFMA kernel from a few rows on, few KV heads the
+    sequence-split kernel up to 128 rows); from three: short caches stay on the split kernel."""
+    def mfma(*a):
+        return C.attention_plan(*a).startswith("k_attention_mfma")
+    for rows in (24, 32, 64, 128, 129):
+        assert mfma(rows, 4096, 64, 64, 128) and mfma(rows, 4096, 64, 64, 64)
+    assert not mfma(4, 4096, 64, 64, 128) and not mfma(1, 4096, 64, 64, 128)
+    assert mfma(96, 1024, 32, 32, 128) and not mfma(32, 256, 32, 32, 128)
+    assert mfma(128, 1024, 64, 32, 128) and not mfma(128, 1024, 16, 8, 128)
+    assert mfma(256, 1024, 8, 8, 256) and not mfma(128, 1024, 8, 4, 256) and mfma(64, 4096, 32, 32, 256)
+    assert not mfma(1024, 0, 1, 1, 128)  # 16 workgroups
+    assert not mfma(96, 0, 32, 8, 128) and mfma(128, 0, 32, 8, 128) and not mfma(48, 0, 64, 8, 128)
+    assert mfma(80, 0, 64, 8, 128) and mfma(96, 0, 32, 8, 256)
+
+
 def test_file_mapping_identity_sees_remaps_and_rewrites(tmp_path):
     """The check made before the device copy of a read-only private file mapping (the engine's
     mmap'd GGUF) is reused: a file unmapped and another mapped at the same address, a rewrite
