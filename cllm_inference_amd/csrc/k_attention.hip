@@ -10,9 +10,10 @@
 //     batch sees pos0 + t + 1 positions).
 //
 // Three attention kernels: k_attention (below; decode, and a few rows over a long cache),
-// k_attention_mfma (many query rows at head_dim 64 and 128, on bf16 MFMA with fp32 operands split
-// in three) and k_attention_mfma_f32 (many query rows at head_dim 256, or over caches of 4 GiB and
-// more, on fp32 MFMA); the layouts of the latter two are described above them.
+// k_attention_mfma (many query rows: at head_dim 64 and 128 on bf16 MFMA with fp32 operands split
+// in three, at 256 on fp32 MFMA) and k_attention_mfma_f32 (many query rows at head_dim 64 and 128
+// over caches of 4 GiB and more, on fp32 MFMA); the layouts of the latter two are described above
+// them.
 //
 // Attention layout. One workgroup per (KV head, query row, sequence split); it serves the
 // n_rep query heads of that KV head, so every K and V row is loaded once for all of them. Its
@@ -530,22 +531,22 @@ hipError_t launch_attention_hd(const float* q, const float* kc, const float* vc,
 
 // ------------------------------------------------------------- many query rows on MFMA
 
-// Prefill attention with fp32's precision: at head_dim 64 and 128 on bf16 MFMA with split operands
-// (k_attention_mfma), at head_dim 256 and over caches of 4 GiB and up on the fp32 matrix cores
-// (k_attention_mfma_f32, v_mfma_f32_16x16x4f32).
+// Prefill attention with fp32's precision: at head_dim 64 and 128 on bf16 MFMA with split operands,
+// at head_dim 256 and over caches of 4 GiB and up on the fp32 matrix cores
+// (v_mfma_f32_16x16x4f32).
 //
 // Split operands. K, V, the queries and the probabilities are sums of three bf16 parts (26 bits);
-// the six largest of the nine part products leave out less than an fp32 product's rounding, and
-// run 2.7 times as fast as the fp32 MFMA. The scores add the leading products apart from the
+// the six largest of the nine part products leave out at most 2^-24 of a product, as much as an fp32
+// product's rounding at most and far less on average, and run 2.7 times as fast as the fp32 MFMA. The scores add the leading products apart from the
 // others (8 rounded additions at head_dim 128, where the fp32 form makes 32), and the P.V products
 // of 32 positions add up from zero, small ones first, before they join the output. Error against
 // 64 bits at 512 rows after 1024 positions (32 + 8 heads of 128): 2.0e-7, the fp32 form's 4.0e-7.
 // Queries are split once into LDS; each wave splits its own K and V rows, beside the MFMAs of the
 // rows before. What bounds it: that VALU work (about 1200 operations beside 192 MFMAs per 32
 // positions and 32 columns) and the loads' way, at two waves per SIMD. MI355X, us, fp32 form against
-// this one: 512 rows after 1024 positions 134.7 / 91, 300 rows 28.7 / 24; 200 rows of 16 + 16
-// heads of 64 13.3 / 12.3. A workgroup with an output that is not finite runs the fp32 form over its blocks (inf * 0
-// appears among the parts where fp32 has inf).
+// this one: 512 rows after 1024 positions 131 / 98, 300 rows 27 / 24.5; 200 rows of 16 + 16 heads
+// of 64 13.3 / 12.3. Columns with an output that is not finite are computed again in fp32 (inf * 0
+// appears among the parts where fp32 has inf; see attention_pass_f32).
 //
 // Columns. A query block is COLS = 16 * CT (row, head) pairs of one KV head: column c is
 // query head c % n_rep of row r0 + c / n_rep, so the n_rep heads of a row and several rows
@@ -596,15 +597,17 @@ __device__ __forceinline__ float quad_reduce(float x) {
 template <int HD, int CT, int W>
 struct AttnLds {
     static constexpr int COLS = 16 * CT, NS = W + 1, PAD = HD + 4;
-    float o[NS][COLS][PAD];
-    float m[NS][COLS], l[NS][COLS];
-    float den[2][COLS];
     int slot_blk[NS];  // the block (0 or 1) whose partial a slot holds, -1: none
+    int bad[2][COLS];  // columns with an output that is not finite
+    float den[2][COLS], max[2][COLS];
+    float m[NS][COLS], l[NS][COLS];
+    alignas(16) float o[NS][COLS][PAD];
 };
 
-// One pass over a workgroup's two row blocks; true where an output of this thread is not finite.
+// One pass over a workgroup's two row blocks; the blocks (bits 0 and 1) where an output of this
+// thread is not finite.
 template <int HD, int CT, int W>
-__device__ __forceinline__ bool attention_pass(
+__device__ __forceinline__ int attention_pass(
     AttnLds<HD, CT, W>& sm, const float* __restrict__ q, const float* __restrict__ kc,
     const float* __restrict__ vc, int n_head, int n_kv, int rows, int pos0, int n_blocks, float scale,
     float* __restrict__ out) {
@@ -642,6 +645,7 @@ __device__ __forceinline__ bool attention_pass(
 
     // the columns of both blocks as three bf16 parts, [block][part][column][HD], 16-byte
     // chunk c of a column at slot c ^ (column & 7)
+    if (threadIdx.x < 2 * COLS) sm.bad[threadIdx.x / COLS][threadIdx.x % COLS] = 0;
     uint8_t* qlds = (uint8_t*)sm.o;
     constexpr int QCOL = HD * 2, QPART = COLS * QCOL;
     static_assert(6 * QPART <= W * COLS * Lds::PAD * 4, "the queries end below the straddling wave's slot");
@@ -879,7 +883,7 @@ __device__ __forceinline__ bool attention_pass(
         den_sm[blk][c] = den;
     }
     __syncthreads();
-    bool bad = false;
+    int bad = 0;
     for (int o4 = threadIdx.x; o4 < 2 * COLS * (HD / 4); o4 += W * 64) {
         const int blk = o4 / (COLS * (HD / 4));
         const int c = (o4 / (HD / 4)) % COLS, d = (o4 % (HD / 4)) * 4;
@@ -897,7 +901,10 @@ __device__ __forceinline__ bool attention_pass(
         }
         const float den = den_sm[blk][c];
         const f32x4 res = f32x4{__fdiv_rn(num.x, den), __fdiv_rn(num.y, den), __fdiv_rn(num.z, den), __fdiv_rn(num.w, den)};
-        bad |= !(fabsf(res.x) < INFINITY && fabsf(res.y) < INFINITY && fabsf(res.z) < INFINITY && fabsf(res.w) < INFINITY);
+        if (!(fabsf(res.x) < INFINITY && fabsf(res.y) < INFINITY && fabsf(res.z) < INFINITY && fabsf(res.w) < INFINITY)) {
+            sm.bad[blk][c] = 1;
+            bad |= 1 << blk;
+        }
         float* orow = out + ((size_t)t * n_head + g * n_rep + c % n_rep) * HD + d;
         orow[0] = res.x;  // out is 4-byte aligned only
         orow[1] = res.y;
@@ -907,65 +914,71 @@ __device__ __forceinline__ bool attention_pass(
     return bad;
 }
 
-// One column in fp32, a wave's lanes over the dims, a position at a time: the rows whose split
-// products are not finite (inf * 0 appears among the parts where fp32 has inf).
+// Positions [p0, p1) of one column, a wave's lanes over the dims (lane + 64 e), four positions at a
+// time, on top of its output o, maximum m and sum l so far.
 template <int HD>
-__device__ __noinline__ void attention_column(const float* qr, const float* kr, const float* vr,
-                                              size_t kv_dim, int L, float scale, float* orow) {
+__device__ __forceinline__ void attention_tail(const float* qr, const float* kr, const float* vr,
+                                               size_t kv_dim, int p0, int p1, float scale,
+                                               float (&o)[HD / 64], float& m, float& l) {
     constexpr int E = HD / 64;
     const int lane = threadIdx.x & 63;
-    float o[E], m = -INFINITY, l = 0.0f;
+    float qv[E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) o[e] = 0.0f;
-    for (int p = 0; p < L; ++p) {
-        float d = 0.0f;
+    for (int e = 0; e < E; ++e) qv[e] = qr[lane + 64 * e];
+    for (int p = p0; p < p1; p += 4) {
+        float s[4], v[4][E], mx = m;
 #pragma unroll
-        for (int e = 0; e < E; ++e) d = __builtin_fmaf(qr[lane + 64 * e], kr[p * kv_dim + lane + 64 * e], d);
+        for (int i = 0; i < 4; ++i) {
+            const size_t at = (size_t)min(p + i, p1 - 1) * kv_dim + lane;
+            s[i] = 0.0f;
 #pragma unroll
-        for (int i = 32; i >= 1; i >>= 1) d += __shfl_xor(d, i, 64);
-        const float s = __fmul_rn(d, scale), mn = fmaxf(m, s);
-        const float pr = s == -INFINITY ? 0.0f : expf(s - mn), cr = m == -INFINITY ? 0.0f : expf(m - mn);
-        l = __builtin_fmaf(l, cr, pr);
+            for (int e = 0; e < E; ++e) {
+                s[i] = __builtin_fmaf(qv[e], kr[at + 64 * e], s[i]);
+                v[i][e] = vr[at + 64 * e];
+            }
+        }
 #pragma unroll
-        for (int e = 0; e < E; ++e) o[e] = __builtin_fmaf(pr, vr[p * kv_dim + lane + 64 * e], o[e] * cr);
-        m = mn;
-    }
+        for (int i = 0; i < 4; ++i) {
 #pragma unroll
-    for (int e = 0; e < E; ++e) orow[lane + 64 * e] = __fdiv_rn(o[e], l);
-}
-
-template <int HD, int CT, int W>
-__global__ __launch_bounds__(W * 64) void k_attention_mfma(
-    const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc,
-    int n_head, int n_kv, int rows, int pos0, int n_blocks, float scale, float* __restrict__ out) {
-    extern __shared__ __align__(16) uint8_t attn_lds[];
-    auto& sm = *(AttnLds<HD, CT, W>*)attn_lds;
-    const bool bad = attention_pass<HD, CT, W>(sm, q, kc, vc, n_head, n_kv, rows, pos0, n_blocks, scale, out);
-    if (!__syncthreads_or(bad)) return;
-    const int g = blockIdx.x % n_kv, pair = blockIdx.x / n_kv, n_rep = n_head / n_kv, rpb = 16 * CT / n_rep;
-    for (int i = threadIdx.x >> 6; i < 2 * rpb * n_rep; i += W) {
-        const int blk = i / (rpb * n_rep), c = i % (rpb * n_rep), b = blk ? n_blocks - 1 - pair : pair;
-        const int t = b * rpb + c / n_rep;
-        if ((blk == 1 && b <= pair) || t >= rows) continue;
-        const size_t at = ((size_t)t * n_head + g * n_rep + c % n_rep) * HD;
-        attention_column<HD>(q + at, kc + (size_t)g * HD, vc + (size_t)g * HD, (size_t)n_kv * HD, pos0 + t + 1,
-                             scale, out + at);
+            for (int j = 32; j >= 1; j >>= 1) s[i] += __shfl_xor(s[i], j, 64);
+            s[i] = p + i < p1 ? __fmul_rn(s[i], scale) : -INFINITY;
+            mx = fmaxf(mx, s[i]);
+        }
+        const float x = expf(m - mx), cr = m == -INFINITY ? 0.0f : x;
+        l *= cr;
+#pragma unroll
+        for (int e = 0; e < E; ++e) o[e] *= cr;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float y = expf(s[i] - mx), pr = s[i] == -INFINITY ? 0.0f : y;
+            l += pr;
+#pragma unroll
+            for (int e = 0; e < E; ++e) o[e] = p + i < p1 ? __builtin_fmaf(pr, v[i][e], o[e]) : o[e];
+        }
+        m = mx;
     }
 }
 
-template <int HD, int CT, int W>
-__global__ __launch_bounds__(W * 64) void k_attention_mfma_f32(
-    const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc,
-    int n_head, int n_kv, int rows, int pos0, int n_blocks, float scale, float* __restrict__ out) {
-    constexpr int COLS = 16 * CT;
+// The fp32 form of a pass. REDO: only the columns of sm.bad, of the blocks of redo (bits 0 and 1).
+// Their MFMA steps then stop at the last whole one that every column of the block sees, and each
+// column's remaining positions (at most 16 and the block's rows) go by themselves: a position that
+// a column does not see is not multiplied by a probability of zero, which an infinite value would
+// make NaN.
+template <int HD, int CT, int W, bool REDO>
+__device__ __forceinline__ void attention_pass_f32(
+    AttnLds<HD, CT, W>& sm, const float* __restrict__ q, const float* __restrict__ kc,
+    const float* __restrict__ vc, int n_head, int n_kv, int rows, int pos0, int n_blocks, float scale,
+    float* __restrict__ out, int redo) {
+    using Lds = AttnLds<HD, CT, W>;
+    constexpr int COLS = Lds::COLS;
     constexpr int DQ = HD / 4;   // K and Q values per lane and row
     constexpr int DV = HD / 16;  // V values per lane and row
-    constexpr int PAD = HD + 4;  // LDS row stride of the partial outputs
-    constexpr int NS = W + 1;    // partial slots: one per wave, one more for the straddling wave
-    __shared__ float o_sm[NS][COLS][PAD];
-    __shared__ float m_sm[NS][COLS], l_sm[NS][COLS];
-    __shared__ float den_sm[2][COLS];
-    __shared__ int slot_blk[NS];  // the block (0 or 1) whose partial a slot holds, -1: none
+    constexpr int NS = Lds::NS;  // partial slots: one per wave, one more for the straddling wave
+    auto& o_sm = sm.o;
+    auto& m_sm = sm.m;
+    auto& l_sm = sm.l;
+    auto& den_sm = sm.den;
+    auto& slot_blk = sm.slot_blk;
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -978,7 +991,9 @@ __global__ __launch_bounds__(W * 64) void k_attention_mfma_f32(
 
     const int blk_row[2] = {pair * rpb, (n_blocks - 1 - pair) * rpb};
     const bool two = n_blocks - 1 - pair > pair;
-    const int len[2] = {pos0 + min(rows, blk_row[0] + rpb), two ? pos0 + min(rows, blk_row[1] + rpb) : 0};
+    const int len[2] = {
+        !REDO ? pos0 + min(rows, blk_row[0] + rpb) : redo & 1 ? (pos0 + blk_row[0] + 1) & ~15 : 0,
+        !two ? 0 : !REDO ? pos0 + min(rows, blk_row[1] + rpb) : redo & 2 ? (pos0 + blk_row[1] + 1) & ~15 : 0};
     const int nA = (len[0] + 15) / 16, T = nA + (len[1] + 15) / 16;
     const int g0 = wave * T / W, g1 = (wave + 1) * T / W;
     if (lane == 0) {
@@ -1100,24 +1115,36 @@ __global__ __launch_bounds__(W * 64) void k_attention_mfma_f32(
         f32x4 sa[CT][2];
         load_k(s0);
         load_v(s0);
-        scores(sa);
-        load_k(s0 + 1);
-        for (int s = s0; s < s1 - 1; ++s) {
-            f32x4 sn[CT][2];
-            scores(sn);        // step s + 1 (K rows requested a step ago)
-            load_k(s + 2);
-            softmax(s, sa);    // step s, beside the score MFMAs
-#pragma unroll
-            for (int i = 0; i < DQ * CT; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-                __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);  // five VALU
+        if constexpr (REDO) {  // (one step at a time: no registers for a second beside the first pass's)
+#pragma unroll 1
+            for (int s = s0; s < s1 - 1; ++s) {
+                scores(sa);
+                load_k(s + 1);
+                softmax(s, sa);
+                pv();
+                load_v(s + 1);
             }
-            pv();
-            load_v(s + 1);     // V rows a step ahead of their P.V MFMAs
+            scores(sa);
+        } else {
+            scores(sa);
+            load_k(s0 + 1);
+            for (int s = s0; s < s1 - 1; ++s) {
+                f32x4 sn[CT][2];
+                scores(sn);        // step s + 1 (K rows requested a step ago)
+                load_k(s + 2);
+                softmax(s, sa);    // step s, beside the score MFMAs
 #pragma unroll
-            for (int ct = 0; ct < CT; ++ct) {
-                sa[ct][0] = sn[ct][0];
-                sa[ct][1] = sn[ct][1];
+                for (int i = 0; i < DQ * CT; ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
+                    __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);  // five VALU
+                }
+                pv();
+                load_v(s + 1);     // V rows a step ahead of their P.V MFMAs
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) {
+                    sa[ct][0] = sn[ct][0];
+                    sa[ct][1] = sn[ct][1];
+                }
             }
         }
         softmax(s1 - 1, sa);
@@ -1155,8 +1182,31 @@ __global__ __launch_bounds__(W * 64) void k_attention_mfma_f32(
             m_sm[z][c] = wgt;
         }
         den_sm[blk][c] = den;
+        if constexpr (REDO) sm.max[blk][c] = M;
     }
     __syncthreads();
+    if constexpr (REDO) {
+        constexpr int E = HD / 64;
+        for (int i = wave; i < 2 * COLS; i += W) {
+            const int blk = i / COLS, c = i % COLS, t = blk_row[blk] + c / n_rep;
+            if (!__builtin_amdgcn_readfirstlane(sm.bad[blk][c])) continue;
+            float o[E], m = sm.max[blk][c], l = den_sm[blk][c];
+#pragma unroll
+            for (int e = 0; e < E; ++e) o[e] = 0.0f;
+            for (int z = 0; z < NS; ++z) {
+                if (slot_blk[z] != blk) continue;
+                const float wgt = m_sm[z][c];
+#pragma unroll
+                for (int e = 0; e < E; ++e) o[e] = __builtin_fmaf(wgt, o_sm[z][c][lane + 64 * e], o[e]);
+            }
+            const size_t at = ((size_t)t * n_head + g * n_rep + c % n_rep) * HD;
+            attention_tail<HD>(q + at, kc + (size_t)g * HD, vc + (size_t)g * HD, kv_dim, len[blk], pos0 + t + 1, scale,
+                               o, m, l);
+#pragma unroll
+            for (int e = 0; e < E; ++e) out[at + lane + 64 * e] = __fdiv_rn(o[e], l);
+        }
+        return;
+    }
     for (int o4 = threadIdx.x; o4 < 2 * COLS * (HD / 4); o4 += W * 64) {
         const int blk = o4 / (COLS * (HD / 4));
         const int c = (o4 / (HD / 4)) % COLS, d = (o4 % (HD / 4)) * 4;
@@ -1181,6 +1231,42 @@ __global__ __launch_bounds__(W * 64) void k_attention_mfma_f32(
     }
 }
 
+// The fp32 form at head_dim 256, the split operands at 64 and 128. A column with an output that is
+// not finite is computed again in fp32 (inf * 0 appears among the parts where fp32 has inf); the
+// others keep their bits. A batch that is NaN throughout takes the time of both forms and of the
+// tails: 512 rows of 32 + 8 heads of 128 after 1024 positions 235 us, 98 when finite (one
+// position at a time and column after column, all columns of the workgroup: 4000).
+template <int HD, int CT, int W>
+__global__ __launch_bounds__(W * 64) void k_attention_mfma(
+    const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc,
+    int n_head, int n_kv, int rows, int pos0, int n_blocks, float scale, float* __restrict__ out) {
+    if constexpr (HD == 256) {
+        __shared__ AttnLds<HD, CT, W> sm;
+        attention_pass_f32<HD, CT, W, false>(sm, q, kc, vc, n_head, n_kv, rows, pos0, n_blocks, scale, out, 0);
+    } else {
+        extern __shared__ __align__(16) uint8_t attn_lds[];
+        auto& sm = *(AttnLds<HD, CT, W>*)attn_lds;
+        const int bad = attention_pass<HD, CT, W>(sm, q, kc, vc, n_head, n_kv, rows, pos0, n_blocks, scale, out);
+        if (!__syncthreads_or(bad)) return;
+        const int redo = (__syncthreads_or(bad & 1) ? 1 : 0) | (__syncthreads_or(bad & 2) ? 2 : 0);
+        attention_pass_f32<HD, CT, W, true>(sm, q, kc, vc, n_head, n_kv, rows, pos0, n_blocks, scale, out, redo);
+    }
+}
+
+// Caches past the split operands' 32-bit offsets.
+template <int HD, int CT, int W>
+__global__ __launch_bounds__(W * 64) void k_attention_mfma_f32(
+    const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc,
+    int n_head, int n_kv, int rows, int pos0, int n_blocks, float scale, float* __restrict__ out) {
+    __shared__ AttnLds<HD, CT, W> sm;
+    attention_pass_f32<HD, CT, W, false>(sm, q, kc, vc, n_head, n_kv, rows, pos0, n_blocks, scale, out, 0);
+}
+
+// Whether the caches are past the split operands' 32-bit offsets.
+bool attention_large_cache(int rows, int pos0, int n_kv, int head_dim) {
+    return ((uint64_t)pos0 + (uint64_t)rows) * (uint64_t)n_kv * (uint64_t)head_dim * sizeof(float) >= (1ull << 32);
+}
+
 template <int HD, int CT, int W>
 hipError_t launch_attention_mfma_hd(const float* q, const float* kc, const float* vc, int rows,
                                     int pos0, int n_head, int n_kv, float* out, hipStream_t stream) {
@@ -1189,25 +1275,25 @@ hipError_t launch_attention_mfma_hd(const float* q, const float* kc, const float
     const int pairs = (n_blocks + 1) / 2;
     const float scale = 1.0f / std::sqrt((float)HD);  // engine.cpp:121, IEEE on the host
     const dim3 grid((unsigned)(n_kv * pairs));
+    int lds = 0;  // of head_dim 256, static
     if constexpr (HD <= 128) {
-        // (the split form's offsets into the caches have 32 bits)
-        if ((uint64_t)(pos0 + rows) * (uint64_t)(n_kv * HD) * sizeof(float) < (1ull << 32)) {
-            constexpr int LDS = sizeof(AttnLds<HD, CT, W>);
-            static_assert(LDS <= 160 * 1024 - 1024, "LDS budget");
-            static std::atomic<bool> attr_set{false};
-            if (!attr_set.load(std::memory_order_acquire)) {
-                const hipError_t e = hipFuncSetAttribute((const void*)k_attention_mfma<HD, CT, W>,
-                                                         hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-                if (e != hipSuccess) return e;
-                attr_set.store(true, std::memory_order_release);
-            }
-            hipLaunchKernelGGL((k_attention_mfma<HD, CT, W>), grid, dim3(W * 64), LDS, stream, q, kc, vc,
-                               n_head, n_kv, rows, pos0, n_blocks, scale, out);
+        if (attention_large_cache(rows, pos0, n_kv, HD)) {
+            hipLaunchKernelGGL((k_attention_mfma_f32<HD, CT, W>), grid, dim3(W * 64), 0, stream, q, kc, vc, n_head,
+                               n_kv, rows, pos0, n_blocks, scale, out);
             return hipGetLastError();
         }
+        lds = sizeof(AttnLds<HD, CT, W>);
+        static_assert(sizeof(AttnLds<HD, CT, W>) <= 160 * 1024, "LDS budget");
+        static std::atomic<bool> attr_set{false};
+        if (!attr_set.load(std::memory_order_acquire)) {
+            const hipError_t e = hipFuncSetAttribute((const void*)k_attention_mfma<HD, CT, W>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+            if (e != hipSuccess) return e;
+            attr_set.store(true, std::memory_order_release);
+        }
     }
-    hipLaunchKernelGGL((k_attention_mfma_f32<HD, CT, W>), grid, dim3(W * 64), 0, stream, q, kc, vc, n_head,
-                       n_kv, rows, pos0, n_blocks, scale, out);
+    hipLaunchKernelGGL((k_attention_mfma<HD, CT, W>), grid, dim3(W * 64), lds, stream, q, kc, vc, n_head, n_kv,
+                       rows, pos0, n_blocks, scale, out);
     return hipGetLastError();
 }
 

@@ -56,6 +56,52 @@ def test_split_attention_non_finite(gpu):
     assert np.array_equal(got[:, 4:], want[:, 4:])
 
 
+@pytest.mark.parametrize("hd,n_head,n_kv", [(64, 8, 2), (128, 8, 2), (64, 4, 4), (128, 14, 2), (128, 5, 5)])
+@pytest.mark.parametrize("rows,pos0", [(96, 20), (130, 0), (40, 300)])
+def test_split_attention_non_finite_columns(gpu, hd, n_head, n_kv, rows, pos0):
+    """Infinities and NaN in queries, keys and values: each column has the infinities and NaNs of the
+    same in 64 bits, and a column that meets none of them keeps its bits, also beside columns of its
+    workgroup that do. (Columns of a row block that holds the first row to see such a value meet it
+    with a probability of zero and are computed again.)"""
+    rng = np.random.default_rng(hd + n_head + rows)
+    L, rep = pos0 + rows, n_head // n_kv
+    q = rng.standard_normal((rows, n_head, hd)).astype(np.float32)
+    kc = rng.standard_normal((L, n_kv, hd)).astype(np.float32)
+    vc = rng.standard_normal((L, n_kv, hd)).astype(np.float32)
+    qb, kb, vb = q.copy(), kc.copy(), vc.copy()
+    touched = np.zeros((rows, n_head), bool)
+    for t, h, val in ((3, 0, np.nan), (rows - 1, n_head - 1, np.inf), (rows // 2, 1, 3.4e38)):
+        qb[t, h, 5] = val
+        touched[t, h] = True
+    # scores of minus infinity (no weight) or infinity (NaN) by the query's sign; a NaN key; values
+    for arr, pos, g, dim, val in ((kb, L - 30, 0, 1, np.inf), (kb, L - 9, 0, 2, np.nan),
+                                  (vb, L - 25, n_kv - 1, 7, np.inf), (vb, L - 21, n_kv - 1, 9, -np.inf),
+                                  (vb, L - 13, n_kv - 1, 11, np.nan), (vb, L - 12, n_kv - 1, 13, 3.4e38)):
+        arr[pos, g, dim] = val
+        first = max(pos - pos0, 0) // (32 // rep) * (32 // rep)
+        touched[first:, g * rep:(g + 1) * rep] = True
+    args = (pos0, n_head, n_kv, hd)
+    gpu.tune("attention_kernel", 2)
+    try:
+        got = gpu.attention_dev(_dev(qb.reshape(rows, -1)), _dev(kb.reshape(L, -1)), _dev(vb.reshape(L, -1)),
+                                *args).cpu().numpy().reshape(rows, n_head, hd)
+        clean = gpu.attention_dev(_dev(q.reshape(rows, -1)), _dev(kc.reshape(L, -1)), _dev(vc.reshape(L, -1)),
+                                  *args).cpu().numpy().reshape(rows, n_head, hd)
+    finally:
+        gpu.tune("attention_kernel")
+    assert touched.any() and not touched.all()
+    assert np.array_equal(got[~touched], clean[~touched])
+    with np.errstate(all="ignore"):
+        want = _attn_ref(qb.reshape(rows, -1), kb.reshape(L, -1), vb.reshape(L, -1), *args).reshape(got.shape)
+    # (scores past 3.4e38 overflow in 32 bits: that column is NaN or one position's values)
+    want[rows // 2, 1] = got[rows // 2, 1]
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want)
+    assert inf.any() and np.array_equal(got[inf], want[inf])
+    fin = np.isfinite(want)
+    np.testing.assert_allclose(got[fin], want[fin], rtol=2e-5, atol=2e-5)
+
+
 @pytest.mark.parametrize("hd,n_head,n_kv", [(128, 4, 2), (256, 4, 2), (64, 2, 1), (256, 8, 1), (256, 4, 1),
                                             (64, 3, 3), (128, 6, 1)])
 def test_decode_attention_edges(gpu, hd, n_head, n_kv):
