@@ -1377,7 +1377,8 @@ void attention_plan_name(int rows, int pos0, int n_head, int n_kv, int head_dim,
                          size_t cap) {
     if (attention_uses_mfma(rows, pos0, n_head, n_kv, head_dim)) {
         const int ct = head_dim == 256 ? 1 : 2, w = head_dim == 256 ? 4 : 8;
-        snprintf(buf, cap, "k_attention_mfma<%d,%d,%d> workgroups=%d", head_dim, ct, w,
+        const bool f32 = head_dim != 256 && attention_large_cache(rows, pos0, n_kv, head_dim);
+        snprintf(buf, cap, "k_attention_mfma%s<%d,%d,%d> workgroups=%d", f32 ? "_f32" : "", head_dim, ct, w,
                  attention_mfma_grid(rows, n_head, n_kv, head_dim).groups);
     } else {
         snprintf(buf, cap, "k_attention<%d> splits=%d", head_dim, attention_splits(rows, pos0, n_kv));

@@ -296,6 +296,12 @@ def test_attention_plans_by_cost():
     assert not mfma(1024, 0, 1, 1, 128)  # 16 workgroups
     assert not mfma(96, 0, 32, 8, 128) and mfma(128, 0, 32, 8, 128) and not mfma(48, 0, 64, 8, 128)
     assert mfma(80, 0, 64, 8, 128) and mfma(96, 0, 32, 8, 256)
+    # caches of 4 GiB and more: the fp32 form, one row short of them: the split operands
+    p = C.attention_plan
+    assert p(64, (1 << 20) - 64, 32, 8, 128).startswith("k_attention_mfma_f32<128,2,8>")
+    assert p(64, (1 << 20) - 65, 32, 8, 128).startswith("k_attention_mfma<128,2,8>")
+    assert p(512, 1 << 20, 64, 16, 64).startswith("k_attention_mfma_f32<64,2,8>")
+    assert p(512, 1 << 20, 16, 4, 256).startswith("k_attention_mfma<256,1,4>")
 
 
 def test_file_mapping_identity_sees_remaps_and_rewrites(tmp_path):

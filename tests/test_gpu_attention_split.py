@@ -102,6 +102,43 @@ def test_split_attention_non_finite_columns(gpu, hd, n_head, n_kv, rows, pos0):
     np.testing.assert_allclose(got[fin], want[fin], rtol=2e-5, atol=2e-5)
 
 
+def test_attention_caches_past_4_gib(gpu):
+    """The fp32 MFMA form at head_dim 64 and 128, which caches of 4 GiB and more take (32-bit offsets
+    in the other), at every number of heads per KV head it lays out differently: the last rows of a
+    long cache against the sequence-split kernel on the same rows and against the same in 64 bits for
+    a few heads. The softmax of 130000 positions: sums of fp32 rounding 2^-24 sqrt(130000) of the
+    mean value, 3e-5 of the largest output."""
+    import torch
+    if torch.cuda.get_device_properties(0).total_memory < 48 << 30:
+        pytest.skip("needs 48 GiB of GPU memory")
+    g = torch.Generator(device="cuda").manual_seed(3)
+    for hd, n_kv in ((128, 64), (64, 128)):
+        L = (1 << 32) // (n_kv * hd * 4) + 117  # 4 GiB and 117 rows
+        k = torch.randn((L, n_kv * hd), device="cuda", generator=g)
+        v = torch.randn((L, n_kv * hd), device="cuda", generator=g)
+        for rep, rows in ((1, 1), (1, 40), (3, 33), (4, 17), (8, 70)):
+            n_head, pos0 = n_kv * rep, L - rows
+            q = torch.randn((rows, n_head * hd), device="cuda", generator=g)
+            print("attention past 4 GiB", hd, n_kv, rep, rows, flush=True)
+            gpu.tune("attention_kernel", 2)
+            try:
+                assert gpu.attention_plan(rows, pos0, n_head, n_kv, hd).startswith(f"k_attention_mfma_f32<{hd}")
+                got = gpu.attention_dev(q, k, v, pos0, n_head, n_kv, hd)
+                gpu.tune("attention_kernel", 1)
+                other = gpu.attention_dev(q, k, v, pos0, n_head, n_kv, hd)
+            finally:
+                gpu.tune("attention_kernel")
+            assert (got - other).abs().max() <= 3e-5 * other.abs().max(), (hd, rep, rows)
+            got = got.view(rows, n_head, hd)
+            for h in (0, n_head // 2, n_head - 1):
+                kv = slice(h // rep * hd, (h // rep + 1) * hd)
+                s = q.view(rows, n_head, hd)[:, h].double() @ k[:, kv].double().T.contiguous() / hd ** 0.5
+                seen = torch.arange(L, device="cuda")[None] <= pos0 + torch.arange(rows, device="cuda")[:, None]
+                want = torch.softmax(s.masked_fill(~seen, float("-inf")), -1) @ v[:, kv].double()
+                assert (got[:, h] - want).abs().max() <= 3e-5 * want.abs().max(), (hd, rep, rows, h)
+        del k, v
+
+
 @pytest.mark.parametrize("hd,n_head,n_kv", [(128, 4, 2), (256, 4, 2), (64, 2, 1), (256, 8, 1), (256, 4, 1),
                                             (64, 3, 3), (128, 6, 1)])
 def test_decode_attention_edges(gpu, hd, n_head, n_kv):
