@@ -11,11 +11,11 @@
 // Split operands. An fp32 value is the sum of three bf16 values of 8 significant bits
 // (rounded to nearest, so the three cover 26 bits), and a bf16 product is exact in the MFMA's
 // fp32 accumulator. With w = w0 + w1 + w2 and x = x0 + x1 + x2, the six products w0 x0, w0 x1,
-// w0 x2, w1 x0, w1 x1, w2 x0 leave out terms below 2^-26 of the product, less than the rounding
-// of an fp32 product (2^-24). At 16 times the rate of the fp32 MFMA, six of them run 2.7 times
-// as fast. F16 weights need two parts (11 bits; five products). A Q3_K weight is d (one per
-// super-block) times the integer scale * code, at most 128 in magnitude and so exact in one
-// bf16: three products, d applied to the super-block's sum.
+// w0 x2, w1 x0, w1 x1, w2 x0 leave out w1 x2 and w2 x1, up to 2^-25 of the product each: at most
+// what rounding an fp32 product takes off (2^-24), and far less on average. At 16 times the rate
+// of the fp32 MFMA, six of them run 2.7 times as fast. F16 weights need two parts (11 bits; five
+// products). A Q3_K weight is d (one per super-block) times the integer scale * code, at most 128
+// in magnitude and so exact in one bf16: three products, d applied to the super-block's sum.
 //
 // Rounding order. The w0 x0 products of 256 elements add up in an accumulator of their own
 // that then goes into the output sum, and the other products, 2^-8 as large, in another: 16
@@ -32,8 +32,11 @@
 //
 // Non-finite values. inf * 0 appears among the split products where fp32 would have inf, and a
 // finite value above the largest bf16 rounds to inf. Any such input makes its outputs
-// non-finite, so outputs that are not finite are computed again, in fp32, by the lane that
-// holds them.
+// non-finite, so a wave's tile (32 rows x 32 tokens) that holds an output that is not finite is
+// computed again on fp32 MFMA, and such outputs take its value. MI355X, us, all finite / one NaN
+// token / all NaN / GEMV: Q3_K 4096 x 4096 at 301 rows 75 / 192 / 324 / 450, F32 at 64 39 / 176 /
+// 169 / 187, Q8_1 at 32 31 / 149 / 147 / 57 (one lane per output, its dot product in series: Q3_K
+// 4100 / 5500).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -122,16 +125,37 @@ struct CfgF {
     static_assert(TASKS * 64 * WN == BM * 8, "whole staging passes");
 };
 
-// One output in fp32: the row's units in order (the outputs the split products could not
-// represent).
+// A 32 x 32 tile in fp32 (v_mfma_f32_32x32x2f32), for the outputs that the split products could not
+// represent: lane (h, r32) decodes unit 2 i + h of weight row wrow and reads the same unit of token
+// row xr, and each pair of elements is one MFMA. Rows and tokens mix in no output, so the others'
+// infinities stay theirs.
 template <uint32_t T>
-__device__ __noinline__ float scalar_dot(const uint8_t* row, int units, const float* xr) {
-    float s = 0.0f;
-    for (int u = 0; u < units; ++u) {
-        float v[32];
-        FUnit<T>::decode(FUnit<T>::load(row, u), u, v);
+__device__ __forceinline__ wf16 tile_f32(const uint8_t* wrow, int units, const float* xr, int h) {
+    wf16 s;
 #pragma unroll
-        for (int e = 0; e < 32; ++e) s = __builtin_fmaf(xr[32 * u + e], v[e], s);
+    for (int r = 0; r < 16; ++r) s[r] = 0.0f;
+    typename FUnit<T>::Raw raw = FUnit<T>::load(wrow, min(h, units - 1));
+    f32x4 xv[8];
+    auto load_x = [&](int u) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) xv[e] = *(const f32x4*)(xr + 32 * u + 4 * e);
+    };
+    load_x(min(h, units - 1));
+#pragma unroll 1
+    for (int u0 = 0; u0 < units; u0 += 2) {
+        const bool in = u0 + h < units;
+        const int next = min(u0 + 2 + h, units - 1);
+        float v[32], xe[32];
+        FUnit<T>::decode(raw, min(u0 + h, units - 1), v);
+#pragma unroll
+        for (int e = 0; e < 32; ++e) {
+            v[e] = in ? v[e] : 0.0f;
+            xe[e] = in ? xv[e / 4][e % 4] : 0.0f;
+        }
+        raw = FUnit<T>::load(wrow, next);  // beside the MFMAs
+        load_x(next);
+#pragma unroll
+        for (int e = 0; e < 32; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(v[e], xe[e], s, 0, 0, 0);
     }
     return s;
 }
@@ -350,14 +374,19 @@ __global__ __launch_bounds__(64 * WN * WK) void k_gemm_f(const uint8_t* __restri
 #pragma unroll
     for (int a = 0; a < MT; ++a) {
         const int t = m0 + 32 * a + r32;
+        bool bad = false;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) bad |= !(fabsf(acc[a][r]) < INFINITY);
+        if (__any(bad)) {
+            const wf16 f = tile_f32<T>(wrow, units, x + (size_t)min(t, m - 1) * k, h);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[a][r] = fabsf(acc[a][r]) < INFINITY ? acc[a][r] : f[r];
+        }
         if (t >= m) continue;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int row = n0 + 8 * (r >> 2) + 4 * h + (r & 3);
-            if (row >= n) continue;
-            float v = acc[a][r];
-            if (!(fabsf(v) < INFINITY)) v = scalar_dot<T>(w + (size_t)row * row_bytes, units, x + (size_t)t * k);
-            y[(size_t)t * n + row] = bias ? v + bv[r] : v;
+            if (row < n) y[(size_t)t * n + row] = bias ? acc[a][r] + bv[r] : acc[a][r];
         }
     }
 }

@@ -62,3 +62,32 @@ def test_split_operand_gemm_non_finite(gpu, orc, qt):
         np.testing.assert_allclose(y[9][fin], ref[9][fin], rtol=1e-5)
     rows = [t for t in range(m) if t not in (1, 4, 7, 9)]
     assert np.array_equal(out[2][rows], beside[rows])
+
+
+@pytest.mark.parametrize("k_units", [1, 9, 16])
+@pytest.mark.parametrize("qt", list(S.FLOAT_DOT_TYPES))
+def test_split_operand_gemm_infinite_weights(gpu, orc, qt, k_units):
+    """Weights that decode to infinity or NaN, in tiles with rows and tokens past the matrix: the
+    reference's infinities and NaNs in their outputs, and no other output changed."""
+    n, m, k = 40, 37, max(S.BLOCK[qt], 32) * k_units
+    w = S.make_weight(qt, n, k, 3)
+    x = S.make_activation(m, k, 4)
+    bad = w.copy()
+    rows = bad.reshape(n, -1)
+    at = {S.Q2_K: 80, S.Q3_K: 108}.get(qt, 0)  # the scale of the row's first block
+    for row, half, single in ((5, 0x7C00, np.inf), (31, 0xFC00, -np.inf), (39, 0x7E00, np.nan)):
+        raw = np.float32(single).tobytes() if qt == S.F32 else np.uint16(half).tobytes()
+        rows[row, at:at + len(raw)] = np.frombuffer(raw, np.uint8)
+    ref = orc.matmul(x, bad, qt, None, k, n, m).reshape(m, n)
+    hit = [5, 31, 39]
+    assert not np.isfinite(ref[:, hit]).any()
+    for knob in (1, 2, 3):
+        gpu.tune("gemm_f", knob)
+        try:
+            y = gpu.matmul_quant_dev(_dev(x), _dev(bad), qt, None, k, n).cpu().numpy()
+            clean = gpu.matmul_quant_dev(_dev(x), _dev(w), qt, None, k, n).cpu().numpy()
+        finally:
+            gpu.tune("gemm_f")
+        assert np.array_equal(y[:, hit], ref[:, hit], equal_nan=True), knob
+        keep = [r for r in range(n) if r not in hit]
+        assert np.array_equal(y[:, keep], clean[:, keep]), knob
