@@ -72,12 +72,18 @@ hipError_t dev_alloc(void** p, size_t bytes) {
 struct DevBuf {
     void* p = nullptr;
     size_t cap = 0;
+    bool held = false;  // a captured graph has its address: not freed when it is outgrown
     // Grows to at least `bytes`. `stream` is synchronised first so no queued kernel still
-    // reads the old allocation.
+    // reads the old allocation. (Sizes double, so held allocations stay below the last one's size.)
     hipError_t ensure(size_t bytes, hipStream_t stream) {
         if (bytes <= cap) return hipSuccess;
         size_t want = cap ? cap : (size_t)1 << 20;
         while (want < bytes) want *= 2;
+        if (held) {
+            p = nullptr;
+            cap = 0;
+            held = false;
+        }
         if (p) {
             hipError_t e = hipStreamSynchronize(stream);
             if (e != hipSuccess) return e;
@@ -167,6 +173,7 @@ struct Workspace {
         v.part_cap = part.cap;
         return e;
     }
+    void hold() { buf.held = part.held = tmp.held = true; }
 };
 
 // A host address range whose bytes have a device copy. Automatic regions are read-only file
@@ -827,7 +834,7 @@ hipError_t run_gemv_f32(uint32_t type, const uint8_t* w, int k, int n, int m, co
 
 // Whether stream s is being captured into a graph: nothing may be allocated then. The routes
 // that calls with rows of k % 256 != 0 took before they had the weight-row kernel allocate less;
-// under capture those calls keep to what is there.
+// under capture those calls keep to what is there (hold: and what they use outlives its growth).
 bool capturing(hipStream_t s) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
@@ -848,10 +855,23 @@ int stream_workspace(DeviceState* st, hipStream_t s, uint32_t type, int k, int n
     if (n > 0 && (use_mfma(type, k, n, m) || use_small(type, k, n, m))) {
         // (without room for its partial sums the weight-row kernel does not split K)
         const size_t pb = part_bytes_for(type, k, n, m);
-        if (k % 256 == 0 || pb <= slot->part.cap || !capturing(s)) HIP_TRY(slot->ensure_part(pb, s));
+        const bool captured = k % 256 != 0 && capturing(s);
+        if (captured) slot->hold();
+        if (!captured || pb <= slot->part.cap) HIP_TRY(slot->ensure_part(pb, s));
     }
     *out = slot.get();
     return CLLM_HIP_OK;
+}
+
+// Whether a call with rows of k % 256 != 0 runs the GEMV although the weight-row kernel would take
+// it: under capture, without room in the stream's workspace for its activation formats and its
+// tmp bytes. (A stream that ran the call before has both, and its captured replays have the eager
+// call's bits.)
+bool captured_without_room(DeviceState* st, hipStream_t s, int k, int m, size_t tmp) {
+    if (k % 256 == 0 || !capturing(s)) return false;
+    std::lock_guard<std::mutex> lk(st->mtx);
+    const auto it = st->dev_ws.find(s);
+    return it == st->dev_ws.end() || !it->second || it->second->buf.cap < act_bytes(k, m) || it->second->tmp.cap < tmp;
 }
 
 // Host-buffer matmul shared by matmul_quant and matmul_quant_batch.
@@ -1091,7 +1111,7 @@ int cllm_hip_gemv_q8_dev(const void* w, uint32_t type, int in_dim, int out_dim, 
     if ((rc = acquire(&st))) return rc;
     hipStream_t s = (hipStream_t)stream;
     if ((!use_mfma(type, in_dim, out_dim, n_rows) && !use_small(type, in_dim, out_dim, n_rows)) ||
-        (in_dim % 256 != 0 && capturing(s))) {
+        captured_without_room(st, s, in_dim, n_rows, 0)) {
         HIP_TRY(launch_gemv(type, (const uint8_t*)w, in_dim, out_dim, n_rows, qs, scales, bsums,
                             bias, y, s));
         return CLLM_HIP_OK;
@@ -1487,15 +1507,15 @@ int cllm_hip_matmul_quant_residual_dev(const float* x, const void* w, uint32_t t
     hipStream_t s = (hipStream_t)stream;
     Workspace* ws = nullptr;
     if ((rc = stream_workspace(st, s, type, in_dim, out_dim, n_rows, &ws))) return rc;
+    const size_t bytes = (size_t)n_rows * out_dim * sizeof(float);
     if (has_kernel(type) &&
         ((!use_mfma(type, in_dim, out_dim, n_rows) && !use_small(type, in_dim, out_dim, n_rows)) ||
-         (in_dim % 256 != 0 && capturing(s)))) {
+         captured_without_room(st, s, in_dim, n_rows, bytes))) {
         // the GEMV adds into y in its epilogue
         HIP_TRY(run_gemv_f32(type, (const uint8_t*)w, in_dim, out_dim, n_rows, x, bias, y, ws->v, s,
                              true));
         return CLLM_HIP_OK;
     }
-    const size_t bytes = (size_t)n_rows * out_dim * sizeof(float);
     {
         std::lock_guard<std::mutex> lk(st->mtx);
         HIP_TRY(ws->tmp.ensure(bytes, s));

@@ -122,3 +122,69 @@ def test_rows_of_whole_blocks_infinite_last_activation_scale(gpu, orc, qt):
     assert np.array_equal(got[3:5], want[3:5], equal_nan=True)
     rest = [t for t in range(m) if t not in (3, 4)]
     np.testing.assert_allclose(got[rest], want[rest], rtol=1e-4, atol=1e-5 * np.abs(want[rest]).max())
+
+
+def _captured(fn, stream):
+    import torch
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=stream):
+        fn()
+    return g
+
+
+def test_rows_of_whole_blocks_captured_after_eager_calls(gpu):
+    """Pre-quantized and residual calls that the stream ran eagerly before have the same bits in the
+    replays of a graph, also after a larger call has outgrown the workspace the graph uses."""
+    import torch
+    qt, n, k, m = S.Q8_0, 300, 2080, 48
+    wd, xd = _dev(S.make_weight(qt, n, k, 1)), _dev(S.make_activation(m, k, 2, outliers=True))
+    big_w, big_x = _dev(S.make_weight(qt, 4096, k, 3)), _dev(S.make_activation(2000, k, 4))
+    y, res, s = torch.zeros((m, n), device="cuda"), torch.zeros((m, n), device="cuda"), torch.cuda.Stream()
+    qs, sc, bs = gpu.quantize_q8_0_dev(xd)
+    assert gpu.matmul_route(qt, k, n, m) == "mfma"
+    torch.cuda.synchronize()
+
+    def calls():
+        gpu.gemv_q8_dev(wd, qt, k, n, qs, sc, bs, y=y)
+        gpu.matmul_quant_residual_dev(xd, wd, qt, None, k, n, res)
+    with torch.cuda.stream(s):
+        calls()
+        eager = (y.clone(), res.clone())
+    g = _captured(calls, s)
+    for rep in range(4):
+        y.zero_(), res.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, eager[0]) and torch.equal(res, eager[1]), rep
+        with torch.cuda.stream(s):  # eager work between the replays; the second one grows the workspace
+            mm = m if rep == 0 else 2000
+            out = torch.zeros((mm, 4096), device="cuda")
+            gpu.matmul_quant_residual_dev(big_x[:mm].contiguous(), big_w, qt, None, k, 4096, out)
+        torch.cuda.synchronize()
+
+
+def test_rows_of_whole_blocks_captured_without_room(gpu, orc):
+    """The same calls captured on a stream whose workspace has no room for them (no pre-quantized call
+    and no residual buffer before) take the GEMV, which allocates nothing."""
+    import torch
+    qt, n, k, m = S.Q8_0, 300, 2080, 48
+    w, x = S.make_weight(qt, n, k, 1), S.make_activation(m, k, 2, outliers=True)
+    wd, xd, s = _dev(w), _dev(x), torch.cuda.Stream()
+    y, res, fresh = torch.zeros((m, n), device="cuda"), torch.zeros((m, n), device="cuda"), torch.cuda.Stream()
+    qs, sc, bs = gpu.quantize_q8_0_dev(xd)
+    with torch.cuda.stream(s):
+        gpu.matmul_quant_dev(xd, wd, qt, None, k, n)  # activations and partial sums, no residual buffer
+    g1 = _captured(lambda: gpu.gemv_q8_dev(wd, qt, k, n, qs, sc, bs, y=y), fresh)
+    g2 = _captured(lambda: gpu.matmul_quant_residual_dev(xd, wd, qt, None, k, n, res), s)
+    want = np.concatenate([gpu.gemv_q8_dev(wd, qt, k, n, qs[t:t + 8].clone(), sc[t:t + 8].clone(),
+                                           bs[t:t + 8].clone()).cpu().numpy() for t in range(0, m, 8)])
+    exact, abs_sum = orc.matmul_f64(x, w, qt, None, k, n, m)
+    yo = orc.matmul(x, w, qt, None, k, n, m)
+    check_close(want, yo, exact, abs_sum, "GEMV")
+    for rep in range(3):
+        y.zero_(), res.zero_()
+        g1.replay(), g2.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(y.cpu().numpy(), want) and np.array_equal(res.cpu().numpy(), want), rep
+        gpu.matmul_quant_dev(xd, wd, qt, None, k, n)
