@@ -41,18 +41,23 @@ def test_rows_of_whole_blocks(gpu, orc, qt, splits):
 
 def test_rows_of_whole_blocks_under_capture(gpu, orc):
     """A captured call with nothing warmed up but the activation workspace, replayed between eager
-    work, equals the eager result."""
+    work, has the bits of an eager call whose K is not split (there is no room for partial sums)."""
     import torch
     qt, n, k, m = S.Q8_0, 300, 2080, 48
     w, x = S.make_weight(qt, n, k, 1), S.make_activation(m, k, 2, outliers=True)
     wd, xd = _dev(w), _dev(x)
     eager = gpu.matmul_quant_dev(xd, wd, qt, None, k, n).clone()
+    gpu.tune("gemm_splits", 1)
+    whole = gpu.matmul_quant_dev(xd, wd, qt, None, k, n).clone()
+    gpu.tune("gemm_splits")
+    assert not torch.equal(whole, eager)  # split by default
     y = torch.zeros((m, n), device="cuda")
     s = torch.cuda.Stream()
     with torch.cuda.stream(s):
-        gpu.quantize_q8_0_dev(xd)
-        gpu.matmul_quant_dev(xd[:15], wd, qt, None, k, n)  # a GEMV batch: no room for split sums
-        gpu.matmul_quant_dev(torch.cat([xd, xd]), wd, S.Q8_0, None, k, 1)
+        # as many activations on a K that is not split: no partial sums are allocated
+        assert "splits=1" in gpu.matmul_plan(qt, 896, 1, 120)
+        gpu.matmul_quant_dev(_dev(S.make_activation(120, 896, 3)), _dev(S.make_weight(qt, 1, 896, 3)), qt,
+                             None, 896, 1)
     torch.cuda.synchronize()
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g, stream=s):
@@ -64,6 +69,7 @@ def test_rows_of_whole_blocks_under_capture(gpu, orc):
         g.replay()
         torch.cuda.synchronize()
         check_close(y.cpu().numpy(), yo, exact, abs_sum, f"replay {rep}")
+        assert torch.equal(y, whole), rep
         again = gpu.matmul_quant_dev(xd, wd, qt, None, k, n)
         assert torch.equal(again, eager)
 
