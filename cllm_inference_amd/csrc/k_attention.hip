@@ -28,7 +28,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 
 #include "device_utils.h"
@@ -1284,13 +1283,9 @@ hipError_t launch_attention_mfma_hd(const float* q, const float* kc, const float
         }
         lds = sizeof(AttnLds<HD, CT, W>);
         static_assert(sizeof(AttnLds<HD, CT, W>) <= 160 * 1024, "LDS budget");
-        static std::atomic<bool> attr_set{false};
-        if (!attr_set.load(std::memory_order_acquire)) {
-            const hipError_t e = hipFuncSetAttribute((const void*)k_attention_mfma<HD, CT, W>,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-            if (e != hipSuccess) return e;
-            attr_set.store(true, std::memory_order_release);
-        }
+        static LdsLimit limit;
+        const hipError_t e = limit.raise((const void*)k_attention_mfma<HD, CT, W>, lds);
+        if (e != hipSuccess) return e;
     }
     hipLaunchKernelGGL((k_attention_mfma<HD, CT, W>), grid, dim3(W * 64), lds, stream, q, kc, vc, n_head, n_kv,
                        rows, pos0, n_blocks, scale, out);

@@ -40,7 +40,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <atomic>
 
 #include "float_units.h"
 #include "ggml_blocks.h"
@@ -395,13 +394,9 @@ template <uint32_t T, int WN, int WK, int MT>
 hipError_t launch_cfg(const uint8_t* w, int k, int n, int m, const float* x, const float* bias,
                       float* y, hipStream_t stream) {
     using C = CfgF<T, WN, WK, MT>;
-    static std::atomic<bool> attr_set{false};
-    if (!attr_set.load(std::memory_order_acquire)) {
-        hipError_t e = hipFuncSetAttribute((const void*)k_gemm_f<T, WN, WK, MT>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
-        if (e != hipSuccess) return e;
-        attr_set.store(true, std::memory_order_release);
-    }
+    static LdsLimit limit;
+    const hipError_t e = limit.raise((const void*)k_gemm_f<T, WN, WK, MT>, C::LDS);
+    if (e != hipSuccess) return e;
     const size_t row_bytes = (size_t)(k / block_elems(T)) * block_bytes(T);
     const unsigned grid = (unsigned)(((n + C::BN - 1) / C::BN) * ((m + C::BM - 1) / C::BM));
     hipLaunchKernelGGL((k_gemm_f<T, WN, WK, MT>), dim3(grid), dim3(C::THREADS), C::LDS, stream, w,

@@ -1360,13 +1360,9 @@ hipError_t launch_b32(const uint8_t* w, int k, int n, int m, const _Float16* qh,
                       const float* bias, float* y, float* part, int* counters, int splits,
                       hipStream_t stream) {
     using C = CfgB<T, W, MT, ANY>;
-    static bool attr_set = false;
-    if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void*)k_gemmw_b32<T, W, MT, ANY, COMP>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
-        if (e != hipSuccess) return e;
-        attr_set = true;
-    }
+    static LdsLimit limit;
+    const hipError_t e = limit.raise((const void*)k_gemmw_b32<T, W, MT, ANY, COMP>, C::LDS);
+    if (e != hipSuccess) return e;
     const uint32_t row_bytes = (uint32_t)(k / 32) * (uint32_t)b32_bytes<T>();
     const int tiles = ((n + C::BN - 1) / C::BN) * ((m + C::BM - 1) / C::BM);
     const int stages = (k + kKS - 1) / kKS;

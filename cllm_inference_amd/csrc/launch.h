@@ -30,6 +30,25 @@ struct Tuning {
 };
 Tuning& tuning();
 
+// Raises a kernel's limit of dynamic LDS once on each device (the attribute belongs to the device
+// that is current when it is set): one static object per kernel, safe from several threads.
+class LdsLimit {
+public:
+    hipError_t raise(const void* kernel, int bytes) {
+        int dev = 0;
+        hipError_t e = hipGetDevice(&dev);
+        if (e != hipSuccess) return e;
+        const uint64_t bit = 1ull << (dev & 63);
+        if (dev < 64 && (done_.load(std::memory_order_acquire) & bit)) return hipSuccess;
+        e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+        if (e == hipSuccess) done_.fetch_or(bit, std::memory_order_release);
+        return e;
+    }
+
+private:
+    std::atomic<uint64_t> done_{0};
+};
+
 // n_blocks consecutive 32-element fp32 blocks -> Q8_0 (qs, fp32 scales, int32 block sums).
 hipError_t launch_quantize_q8_0(const float* x, int64_t n_blocks, int8_t* qs, float* scales,
                                 int32_t* bsums, hipStream_t stream);
