@@ -608,6 +608,12 @@ bool gemm_forced();
 // kernel instead: Q5_K 14336x4096 at 20 / 24 / 28 / 32 rows 25.9 / 26.5 / 26.5 / 27.0 us
 // against 28.2 / 28.6 / 28.8 / 29.6 (Q4_K 4096x4096 and 1024x4096 stay faster here: 15.3
 // against 18.9 us at 32 rows).
+// All of these lines, here and below, were measured before the weight-row kernel's items were
+// pipelined. Since then, us, this kernel against it, at 32 / 48 / 64 rows: Q8_0 14336x4096 27.3 /
+// 35.8 / 43.2 against 26.4 / 34.3 / 35.8, 4096x14336 29.8 / 44.9 / 57.6 against 31.7 / 41.0 / 42.1,
+// 4096x4096 14.9 / 17.6 / 19.3 against 20.3 / 25.8 / 27.1; Q4_0 14336x4096 26.1 / 35.0 / 42.0 against
+// 25.0 / 32.3 / 33.8; Q4_K 4096x14336 at 20 rows 28.8 against 28.3. So from 48 rows on matrices of
+// 32 M weights or more the lines lie up to 20 % too high; elsewhere they hold.
 constexpr int kSmallMinRows = 8;
 constexpr int kSmallMaxN = 8192;
 

@@ -46,7 +46,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // to the second tensor x2 (the keys), so the queries and keys of a layer turn in one launch. The
 // head_dim / 2 angles of the row are formed once per workgroup (a power, a cosine and a sine each)
 // and turn all of its heads: with a workgroup per head that arithmetic, on a quarter of the lanes,
-// took 11.8 us for 512 rows of 32 + 8 heads of 128; now 6.2 (20 MB moved).
+// took 11.8 us for 512 rows of 32 + 8 heads of 128; now 6.2 (20 MB moved). From ten heads on the
+// angles no longer show there (2 / 4 / 10 / 20 heads per workgroup, a call every 10.7 / 8.0 / 7.5 /
+// 7.4 us); 2048 rows take 34 / 24 / 17.7 / 15.6.
 constexpr int kRopeHeads = 10;
 __global__ __launch_bounds__(256) void k_rope_neox(float* __restrict__ x, int n_heads,
                                                    float* __restrict__ x2, int n_heads2,
@@ -1309,8 +1311,8 @@ hipError_t launch_rope_neox(float* x, int rows, int n_heads, float* x2, int n_he
 }
 
 size_t attention_workspace_bytes(int rows, int n_head, int head_dim) {
-    // at most 1024 / (n_kv * rows) + 1 splits, n_kv >= 1
-    const size_t splits = (size_t)(1024 / std::max(rows, 1) + 1);
+    // attention_splits: at most 512 / (n_kv * rows) + 1 splits, n_kv >= 1
+    const size_t splits = (size_t)(512 / std::max(rows, 1) + 1);
     return kAttnCounters * sizeof(int) + (size_t)rows * n_head * splits * (head_dim + 4) * sizeof(float);
 }
 

@@ -428,7 +428,8 @@ int cus() {
 // The tile shape for a batch (1: 128 x 64, K on 2 waves; 2: 64 x 32, K on 2; 3: 32 x 32, K on
 // 4), or 0 where the GEMV is faster, by the time each would take. A stage (64 WK elements)
 // takes a workgroup about the same time however many run beside it, up to one per CU; two or
-// three of shape 2 share a CU. MI355X, cold weights, us (GEMV / shapes 1 / 2 / 3):
+// three of shape 2 share a CU. The constants fit the measurements below and their like; a shape
+// has to beat the GEMV by 3 us of that estimate. MI355X, cold weights, us (GEMV / shapes 1 / 2 / 3):
 //   Q3_K 4096 x 4096,  16 rows:  26.7 /  66 /  37 /  28     F32 4096 x 4096, 301 rows:  810 / 94 / 124 / 167
 //                      32:       55.5 /  66 /  38 /  29     Q4_1 4096 x 4096, 301:      476 / 85 /  93 / 142
 //                      64:        100 /  66 /  38 /  30     Q2_K 14336 x 4096, 16:       73 / 86 /  42 /  56

@@ -862,8 +862,15 @@ __global__ __launch_bounds__(64 * W) void k_gemmw_q6k(const uint8_t* __restrict_
 //   y += dx * (d * I)
 // costs two VALU operations per output and block (d belongs to the weight row, dx to the
 // token). A stage is 4 blocks (128 elements); the rows' stage bytes (4 blocks of 34 / 18 / 22
-// bytes, 4-byte aligned because k % 256 == 0) arrive by 4-byte direct-to-LDS loads in the
+// bytes, 4-byte aligned where k % 128 == 0) arrive by 4-byte direct-to-LDS loads in the
 // blocks' own layout, and each lane realigns its 2-byte-aligned fields from 4-byte LDS reads.
+//
+// Rows that are no multiple of 256 long. COMP (any of them): the sums of stage pairs join the
+// output with the rounding carried on (one chain was 9.9e-8 off the 64-bit result at K = 896, the
+// GEMV 7.0e-8, this 6.5e-8). ANY (no multiple of 128): rows start at multiples of 2 bytes, so an
+// LDS row is the window from the dword below, and the last stage has one to three blocks. Its
+// 128 x 64 tiles of Q8_0 and Q5_0 need more than 256 registers and run one wave per SIMD where the
+// others run two: Q8_0 12000 x 8224 at 48 rows takes 88 us, Q4_0 58.
 template <uint32_t T>
 constexpr int b32_bytes() { return T == T_Q8_0 ? Q8_0_BYTES : T == T_Q4_0 ? Q4_0_BYTES : Q5_0_BYTES; }
 

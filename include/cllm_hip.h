@@ -198,7 +198,9 @@ int cllm_hip_matmul_quant_dev(const float* x, const void* w, uint32_t type, cons
  * (quantized activations, the MFMA formats, split-K partial sums) is carved from a fixed
  * array of cllm_hip_static_scratch_bytes() (64 MiB) per GPU, held from library load to process
  * end, and nothing is allocated or freed (call cllm_hip_init first: it builds the per-device
- * state once). A batch whose scratch exceeds the array fails with CLLM_HIP_E_ARG (M = 512
+ * state once). Where only the split-K partial sums of rows that are no multiple of 256 long would
+ * not fit, K is not split (another order of additions than cllm_hip_matmul_quant_dev's). A batch
+ * whose scratch exceeds the array otherwise fails with CLLM_HIP_E_ARG (M = 512
  * rows of 14336 need ~27 MB; split larger batches). Every call on one GPU shares that GPU's
  * array, which keeps the last call's contents. Calls on one stream are ordered by it; a call
  * on another stream while the last eager call's work may still be running fails with
