@@ -30,12 +30,17 @@
 // (16-byte chunks swizzled by token: a wave's fragment reads spread over all banks), two
 // stages of 64 WK elements in turn.
 //
+// Small values. The matrix cores take bf16 values below 2^-126 for zero, which the lower parts of
+// fp32 values below 2^-101 are (1.1e-6 off at 2^-115, 3.6e-2 at 2^-130). So the activations, and fp32
+// weights, are split times 2^26, and the sums go back by as much: exact, at any size. (The other
+// types' weights have binary16 scales, 2^-24 and up.)
+//
 // Non-finite values. inf * 0 appears among the split products where fp32 would have inf, and a
-// finite value above the largest bf16 rounds to inf. Any such input makes its outputs
+// finite value that is above the largest bf16 times 2^26 rounds to inf. Any such input makes its outputs
 // non-finite, so a wave's tile (32 rows x 32 tokens) that holds an output that is not finite is
 // computed again on fp32 MFMA, and such outputs take its value. MI355X, us, all finite / one NaN
-// token / all NaN / GEMV: Q3_K 4096 x 4096 at 301 rows 75 / 192 / 324 / 450, F32 at 64 39 / 176 /
-// 169 / 187, Q8_1 at 32 31 / 149 / 147 / 57 (one lane per output, its dot product in series: Q3_K
+// token / all NaN / GEMV: Q3_K 4096 x 4096 at 301 rows 75 / 199 / 326 / 450, F32 at 64 39 / 168 /
+// 166 / 187, Q8_1 at 32 31 / 139 / 138 / 57 (one lane per output, its dot product in series: Q3_K
 // 4100 / 5500).
 #include <hip/hip_runtime.h>
 
@@ -110,6 +115,8 @@ template <> struct GUnit<T_Q3_K> {
     }
 };
 
+constexpr float kUp = 0x1p26f;  // what operands are multiplied with before they are split
+
 template <uint32_t T, int WN, int WK, int MT>
 struct CfgF {
     static constexpr int THREADS = 64 * WN * WK;
@@ -126,8 +133,9 @@ struct CfgF {
 
 // A 32 x 32 tile in fp32 (v_mfma_f32_32x32x2f32), for the outputs that the split products could not
 // represent: lane (h, r32) decodes unit 2 i + h of weight row wrow and reads the same unit of token
-// row xr, and each pair of elements is one MFMA. Rows and tokens mix in no output, so the others'
-// infinities stay theirs.
+// row xr, and each pair of elements is one MFMA; 32 elements add up from zero before they join the
+// tile (one chain over 1024 was 5.6e-7 off the 64-bit sums, this 1.5e-7, the GEMV 1.2e-7). Rows and
+// tokens mix in no output, so the others' infinities stay theirs.
 template <uint32_t T>
 __device__ __forceinline__ wf16 tile_f32(const uint8_t* wrow, int units, const float* xr, int h) {
     wf16 s;
@@ -154,7 +162,13 @@ __device__ __forceinline__ wf16 tile_f32(const uint8_t* wrow, int units, const f
         raw = FUnit<T>::load(wrow, next);  // beside the MFMAs
         load_x(next);
 #pragma unroll
-        for (int e = 0; e < 32; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(v[e], xe[e], s, 0, 0, 0);
+        for (int e = 0; e < 32; e += 16) {
+            wf16 c = {};
+#pragma unroll
+            for (int i = 0; i < 16; ++i) c = __builtin_amdgcn_mfma_f32_32x32x2f32(v[e + i], xe[e + i], c, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] += c[r];
+        }
     }
     return s;
 }
@@ -167,6 +181,7 @@ __global__ __launch_bounds__(64 * WN * WK) void k_gemm_f(const uint8_t* __restri
                                                          float* __restrict__ y) {
     using C = CfgF<T, WN, WK, MT>;
     constexpr int PW = wparts<T>();
+    constexpr float kDown = T == T_F32 ? 1.0f / kUp / kUp : 1.0f / kUp;
     extern __shared__ __align__(16) uint8_t lds[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -213,11 +228,12 @@ __global__ __launch_bounds__(64 * WN * WK) void k_gemm_f(const uint8_t* __restri
     auto store_x = [&](int s, uint8_t* st) {
 #pragma unroll
         for (int i = 0; i < C::TASKS; ++i) {
-            const bool in = xu[i] + 8 * WK * (s >> 2) + (s & 3) < units;  // zeros past K
+            // zeros past K (times the token's last values: where those are infinite, so are its outputs)
+            const float up = xu[i] + 8 * WK * (s >> 2) + (s & 3) < units ? kUp : 0.0f;
             const f32x4 lo4 = xr[i][0], hi4 = xr[i][1];
             float v[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = in ? v[e] : 0.0f;
+            for (int e = 0; e < 8; ++e) v[e] *= up;
             wbf8 p[3];
             split8<3>(v, p);
 #pragma unroll
@@ -238,6 +254,10 @@ __global__ __launch_bounds__(64 * WN * WK) void k_gemm_f(const uint8_t* __restri
     auto frag = [&](int j, int q, wbf8 (&a)[PW]) {
         float wv[32];
         GUnit<T>::decode(raw, GUnit<T>::HALF ? 4 * h + j : 0, wv);
+        if constexpr (T == T_F32) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) wv[8 * q + e] *= kUp;
+        }
         split8<PW>(wv + 8 * q, a);
     };
     wbf8 afr[2][PW];
@@ -379,7 +399,10 @@ __global__ __launch_bounds__(64 * WN * WK) void k_gemm_f(const uint8_t* __restri
         if (__any(bad)) {
             const wf16 f = tile_f32<T>(wrow, units, x + (size_t)min(t, m - 1) * k, h);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[a][r] = fabsf(acc[a][r]) < INFINITY ? acc[a][r] : f[r];
+            for (int r = 0; r < 16; ++r) acc[a][r] = fabsf(acc[a][r]) < INFINITY ? acc[a][r] * kDown : f[r];
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[a][r] *= kDown;
         }
         if (t >= m) continue;
 #pragma unroll

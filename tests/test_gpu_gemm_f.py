@@ -91,3 +91,35 @@ def test_split_operand_gemm_infinite_weights(gpu, orc, qt, k_units):
         assert np.array_equal(y[:, hit], ref[:, hit], equal_nan=True), knob
         keep = [r for r in range(n) if r not in hit]
         assert np.array_equal(y[:, keep], clean[:, keep]), knob
+
+
+@pytest.mark.parametrize("qt,w_exp,x_exp", [(S.F32, -120, 115), (S.F32, 112, -118), (S.F32, -60, -55),
+                                            (S.F16, 0, -118), (S.Q4_1, 0, -118), (S.Q8_1, 0, -118),
+                                            (S.Q2_K, 0, -115), (S.Q3_K, 0, -115), (S.Q5_1, 0, 90)])
+def test_split_operand_gemm_small_and_large_values(gpu, qt, w_exp, x_exp):
+    """Weights and activations far from 1, whose lower bf16 parts the matrix cores would take for zero:
+    as near to the 64-bit sums as batches around 1. (Values of 2^-6 to 1 before the scaling: none is
+    below the smallest normal fp32. 512 terms of random sign: sums of fp32 rounding, 3e-7 of the
+    result's norm at most; without the scaling 1e-5 and up.)"""
+    import torch
+    n, m, k = 96, 40, 512
+    rng = np.random.default_rng(qt)
+    x = (rng.uniform(2.0 ** -6, 1, (m, k)) * rng.choice([-1, 1], (m, k))).astype(np.float32)
+    if qt == S.F32:
+        w = (rng.uniform(2.0 ** -6, 1, (n, k)) * rng.choice([-1, 1], (n, k))).astype(np.float32)
+        full = w.astype(np.float64)
+        w = (w * np.float32(2.0) ** w_exp).view(np.uint8).reshape(-1)
+    else:
+        w = S.make_weight(qt, n, k, 3)
+        full = gpu.dequantize_rows_dev(_dev(w), qt, k, torch.arange(n, device="cuda", dtype=torch.int32))
+        full = full.double().cpu().numpy().reshape(n, k)
+    want = x.astype(np.float64) @ full.T
+    xs = _dev(x * np.float32(2.0) ** x_exp)
+    for knob in (1, 2, 3):
+        gpu.tune("gemm_f", knob)
+        try:
+            y = gpu.matmul_quant_dev(xs, _dev(w), qt, None, k, n).double().cpu().numpy()
+        finally:
+            gpu.tune("gemm_f")
+        err = y * 2.0 ** -(w_exp + x_exp) - want
+        assert np.linalg.norm(err) <= 3e-7 * np.linalg.norm(want), (knob, np.linalg.norm(err) / np.linalg.norm(want))
