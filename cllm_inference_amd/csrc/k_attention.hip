@@ -547,7 +547,8 @@ hipError_t launch_attention_hd(const float* q, const float* kc, const float* vc,
 // positions and 32 columns) and the loads' way, at two waves per SIMD. MI355X, us, fp32 form against
 // this one: 512 rows after 1024 positions 131 / 98, 300 rows 27 / 24.5; 200 rows of 16 + 16 heads
 // of 64 13.3 / 12.3. Columns with an output that is not finite are computed again in fp32 (inf * 0
-// appears among the parts where fp32 has inf; see attention_pass_f32).
+// appears among the parts where fp32 has inf; see attention_pass_f32), and so are those with one
+// of less than 2^-90 (see kQueryUp).
 //
 // Columns. A query block is COLS = 16 * CT (row, head) pairs of one KV head: column c is
 // query head c % n_rep of row r0 + c / n_rep, so the n_rep heads of a row and several rows
@@ -599,14 +600,20 @@ template <int HD, int CT, int W>
 struct AttnLds {
     static constexpr int COLS = 16 * CT, NS = W + 1, PAD = HD + 4;
     int slot_blk[NS];  // the block (0 or 1) whose partial a slot holds, -1: none
-    int bad[2][COLS];  // columns with an output that is not finite
+    int bad[2][COLS];  // columns to compute again
     float den[2][COLS], max[2][COLS];
     float m[NS][COLS], l[NS][COLS];
     alignas(16) float o[NS][COLS][PAD];
 };
 
+// The matrix cores take bf16 values below 2^-126 for zero, which the lower parts of fp32 values below
+// 2^-101 are. The queries are split times this factor: then none is, keys lose less than 2^-53 of a
+// score, and queries from 2^66 and scores from 2^66 on overflow and are computed again in fp32.
+constexpr float kQueryUp = 0x1p62f;
+
 // One pass over a workgroup's two row blocks; the blocks (bits 0 and 1) where an output of this
-// thread is not finite.
+// thread is not finite, or so small that lower parts of the values were lost (below 2^-90; values
+// that are all below 2^-126 come out as zero).
 template <int HD, int CT, int W>
 __device__ __forceinline__ int attention_pass(
     AttnLds<HD, CT, W>& sm, const float* __restrict__ q, const float* __restrict__ kc,
@@ -659,7 +666,7 @@ __device__ __forceinline__ int attention_pass(
             const f32x4 v0 = *(const f32x4*)qr, v1 = *(const f32x4*)(qr + 4);
             float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = valid ? v[e] : 0.0f;
+            for (int e = 0; e < 8; ++e) v[e] = valid ? v[e] * kQueryUp : 0.0f;
             wbf8 p[3];
             split8<3>(v, p);
 #pragma unroll
@@ -788,7 +795,7 @@ __device__ __forceinline__ int attention_pass(
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     const int p = s * 32 + (e < 4 ? 0 : 16) + 4 * quad + (e & 3);
-                    sv[e] = p <= lim[ct] ? __fmul_rn(sc[e >> 2][ct][e & 3], scale) : -INFINITY;
+                    sv[e] = p <= lim[ct] ? __fmul_rn(sc[e >> 2][ct][e & 3], scale / kQueryUp) : -INFINITY;
                     mx = fmaxf(mx, sv[e]);
                 }
                 mx = quad_reduce<true>(mx);
@@ -902,7 +909,9 @@ __device__ __forceinline__ int attention_pass(
         }
         const float den = den_sm[blk][c];
         const f32x4 res = f32x4{__fdiv_rn(num.x, den), __fdiv_rn(num.y, den), __fdiv_rn(num.z, den), __fdiv_rn(num.w, den)};
-        if (!(fabsf(res.x) < INFINITY && fabsf(res.y) < INFINITY && fabsf(res.z) < INFINITY && fabsf(res.w) < INFINITY)) {
+        // (a magnitude between them, or zero; NaN is neither)
+        const auto sound = [](float v) { return (fabsf(v) < INFINITY && fabsf(v) >= 0x1p-90f) || v == 0.0f; };
+        if (!(sound(res.x) && sound(res.y) && sound(res.z) && sound(res.w))) {
             sm.bad[blk][c] = 1;
             bad |= 1 << blk;
         }

@@ -102,6 +102,43 @@ def test_split_attention_non_finite_columns(gpu, hd, n_head, n_kv, rows, pos0):
     np.testing.assert_allclose(got[fin], want[fin], rtol=2e-5, atol=2e-5)
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("q_exp,k_exp,v_exp", [(-116, 114, 0), (114, -116, 0), (0, 0, -116), (0, 0, 110),
+                                               (-60, 60, -95)])
+def test_split_attention_small_and_large_values(gpu, hd, q_exp, k_exp, v_exp):
+    """Queries, keys and values far from 1, whose lower bf16 parts the matrix cores would take for zero:
+    as near to the same in 64 bits as values around 1 (2e-6 of the largest output; without a measure
+    against it 1e-5 and up). (Values of 2^-6 to 2 before the scaling: none is below the smallest
+    normal fp32.)"""
+    rng = np.random.default_rng(hd + abs(v_exp))
+    n_head, n_kv, rows, pos0 = 8, 2, 70, 50
+    def draw(r, c):
+        return (rng.uniform(2.0 ** -6, 2, (r, c)) * rng.choice([-1, 1], (r, c))).astype(np.float32)
+    q, k, v = draw(rows, n_head * hd), draw(pos0 + rows, n_kv * hd), draw(pos0 + rows, n_kv * hd)
+    two = np.float32(2.0)
+    gpu.tune("attention_kernel", 2)
+    try:
+        got = gpu.attention_dev(_dev(q * two ** q_exp), _dev(k * two ** k_exp), _dev(v * two ** v_exp), pos0,
+                                n_head, n_kv, hd).cpu().numpy().astype(np.float64) * 2.0 ** -v_exp
+    finally:
+        gpu.tune("attention_kernel")
+    want = _attn_ref(q * two ** (q_exp + k_exp), k, v, pos0, n_head, n_kv, hd)
+    assert (np.abs(got - want) <= 2e-6 * np.abs(want).max()).all(), np.abs(got - want).max()
+
+
+def test_split_attention_zero_values(gpu):
+    """Value dims that are all zero (padding) stay zero."""
+    rng = np.random.default_rng(1)
+    q, k, v = (rng.standard_normal((r, c * 128)).astype(np.float32) for r, c in ((64, 8), (200, 2), (200, 2)))
+    v.reshape(200, 2, 128)[:, :, 80:] = 0.0
+    gpu.tune("attention_kernel", 2)
+    try:
+        got = gpu.attention_dev(_dev(q), _dev(k), _dev(v), 136, 8, 2, 128).cpu().numpy().reshape(64, 8, 128)
+    finally:
+        gpu.tune("attention_kernel")
+    assert not got[:, :, 80:].any() and (got[:, :, :80] != 0).all()
+
+
 def test_attention_caches_past_4_gib(gpu):
     """The fp32 MFMA form at head_dim 64 and 128, which caches of 4 GiB and more take (32-bit offsets
     in the other), at every number of heads per KV head it lays out differently: the last rows of a
