@@ -173,7 +173,7 @@ struct Workspace {
         v.part_cap = part.cap;
         return e;
     }
-    void hold() { buf.held = part.held = tmp.held = true; }
+    void hold() { buf.held = part.held = att.held = tmp.held = true; }
 };
 
 // A host address range whose bytes have a device copy. Automatic regions are read-only file
@@ -840,7 +840,7 @@ hipError_t run_gemv_f32(uint32_t type, const uint8_t* w, int k, int n, int m, co
 
 // Whether stream s is being captured into a graph: nothing may be allocated then. The routes
 // that calls with rows of k % 256 != 0 took before they had the weight-row kernel allocate less;
-// under capture those calls keep to what is there (hold: and what they use outlives its growth).
+// under capture those calls keep to what is there.
 bool capturing(hipStream_t s) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
@@ -850,20 +850,21 @@ bool capturing(hipStream_t s) {
     return cap != hipStreamCaptureStatusNone;
 }
 
-// The per-stream workspace of the device entry points, grown to an m x k batch and to the
+// The per-stream workspace of the device entry points (a captured graph's share of it outlives its
+// growth by later calls), grown to an m x k batch and to the
 // split-K region of an n-row MFMA call on it (n = 0: none).
 int stream_workspace(DeviceState* st, hipStream_t s, uint32_t type, int k, int n, int m,
                      Workspace** out) {
     std::lock_guard<std::mutex> lk(st->mtx);
     auto& slot = st->dev_ws[s];
     if (!slot) slot = std::make_unique<Workspace>();
+    const bool captured = capturing(s);
+    if (captured) slot->hold();
     HIP_TRY(slot->ensure(k, m, s));
     if (n > 0 && (use_mfma(type, k, n, m) || use_small(type, k, n, m))) {
         // (without room for its partial sums the weight-row kernel does not split K)
         const size_t pb = part_bytes_for(type, k, n, m);
-        const bool captured = k % 256 != 0 && capturing(s);
-        if (captured) slot->hold();
-        if (!captured || pb <= slot->part.cap) HIP_TRY(slot->ensure_part(pb, s));
+        if (k % 256 == 0 || !captured || pb <= slot->part.cap) HIP_TRY(slot->ensure_part(pb, s));
     }
     *out = slot.get();
     return CLLM_HIP_OK;
@@ -1348,6 +1349,7 @@ int cllm_hip_matmul_mfma_dev(uint32_t type, int in_dim, int n_mats, const void* 
         auto& slot = st->dev_ws[s];
         if (!slot) slot = std::make_unique<Workspace>();
         ws = slot.get();
+        if (capturing(s)) ws->hold();
     }
     const uint8_t* const* wb = (const uint8_t* const*)w;
     if (gemmw_multi_supported(type, n_mats)) {

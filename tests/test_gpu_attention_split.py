@@ -200,3 +200,32 @@ def test_decode_attention_edges(gpu, hd, n_head, n_kv):
                 assert (err <= 2e-6 * np.maximum(scale, 1e-3)).all(), (pos0, rows, err.max())
     finally:
         gpu.tune("attention_kernel")
+
+
+def test_captured_attention_outlives_its_workspace(gpu):
+    """A batch of one head per KV head on the sequence-split kernel, captured after an eager call, keeps
+    its bits in replays after a larger call on the stream has outgrown the split partials' workspace."""
+    import torch
+    hd, heads, rows, pos0 = 128, 8, 64, 1024
+    assert gpu.attention_plan(rows, pos0, heads, heads, hd).startswith("k_attention<")
+    g = torch.Generator(device="cuda").manual_seed(2)
+    q, k, v = (torch.randn((r, heads * hd), device="cuda", generator=g) for r in (rows, pos0 + rows, pos0 + rows))
+    big = torch.randn((2048, 32 * hd), device="cuda", generator=g)
+    out, s = torch.zeros_like(q), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        eager = gpu.attention_dev(q, k, v, pos0, heads, heads, hd).clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        gpu.attention_dev(q, k, v, pos0, heads, heads, hd, out=out)
+    for rep in range(4):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager), rep
+        with torch.cuda.stream(s):  # the workspace is sized by rows and heads: 2048 rows outgrow it
+            n = 64 if rep == 0 else 2048
+            gpu.attention_dev(big[:n].contiguous(), big[:n, :8 * hd].contiguous(), big[:n, :8 * hd].contiguous(),
+                              0, 32, 8, hd)
+        torch.cuda.synchronize()
