@@ -393,23 +393,27 @@ __global__ __launch_bounds__(64 * WN * WK) void k_gemm_f(const uint8_t* __restri
 #pragma unroll
     for (int a = 0; a < MT; ++a) {
         const int t = m0 + 32 * a + r32;
-        bool bad = false;
+        // (times kDown is exact, so one FMA rounds as the bias's addition does)
+        auto store = [&](int r, float v, float down) {
+            const int row = n0 + 8 * (r >> 2) + 4 * h + (r & 3);
+            if (row < n) y[(size_t)t * n + row] = bias ? __builtin_fmaf(v, down, bv[r]) : v * down;
+        };
+        float nan = 0.0f;  // once an output is not finite
 #pragma unroll
-        for (int r = 0; r < 16; ++r) bad |= !(fabsf(acc[a][r]) < INFINITY);
-        if (__any(bad)) {
+        for (int r = 0; r < 16; ++r) nan = __builtin_fmaf(acc[a][r], 0.0f, nan);
+        if (__any(nan != 0.0f)) {
             const wf16 f = tile_f32<T>(wrow, units, x + (size_t)min(t, m - 1) * k, h);
+            if (t >= m) continue;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[a][r] = fabsf(acc[a][r]) < INFINITY ? acc[a][r] * kDown : f[r];
-        } else {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[a][r] *= kDown;
+            for (int r = 0; r < 16; ++r) {
+                const bool fin = fabsf(acc[a][r]) < INFINITY;
+                store(r, fin ? acc[a][r] : f[r], fin ? kDown : 1.0f);
+            }
+            continue;
         }
         if (t >= m) continue;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int row = n0 + 8 * (r >> 2) + 4 * h + (r & 3);
-            if (row < n) y[(size_t)t * n + row] = bias ? acc[a][r] + bv[r] : acc[a][r];
-        }
+        for (int r = 0; r < 16; ++r) store(r, acc[a][r], kDown);
     }
 }
 
